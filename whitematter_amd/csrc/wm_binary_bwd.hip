@@ -4,7 +4,7 @@
 // The reference closures (core/tensor.cpp:956-976 and the same loop in
 // sub/mul/div/pow/max/min) walk the output in row-major order and scatter
 // "grad[src_idx] += contribution" one element at a time.  Here the output is
-// folded to the fewest dims (as in the forward) and three layouts get their
+// folded to the fewest dims (as in the forward) and these layouts get their
 // own kernels:
 //   flat    both operands have the output's shape: one fused elementwise pass;
 //   colsum  one operand is full [R,C], the other a row vector [1,C]: column
@@ -12,7 +12,10 @@
 //           fixed-order second pass (c1 bias grad, c2 r.grad, c5 g.grad);
 //   rowsum  one operand is full, the other a column vector [R,1] (or a
 //           scalar): one wave per (row, column chunk), DPP wave reduction,
-//           then a fixed-order second pass when a row is split (c2 c.grad).
+//           then a fixed-order second pass when a row is split (c2 c.grad);
+//   cols    [O,R,C] with [O,1,C], and the row vectors colsum does not take
+//           (short, ragged or unaligned rows);
+//   channel [O,K,I] with [1,K,1] (a convolution's bias).
 // Everything else goes through a generic kernel: one thread per operand
 // element, summing its contributions in the reference's row-major order.
 // Every path is deterministic: no atomics, fixed partition, fixed order.
@@ -36,8 +39,9 @@ template <int OP>
 __global__ void __launch_bounds__(kBlock) bwd_flat_kernel(const float* __restrict__ g, const float* __restrict__ a,
                                                            const float* __restrict__ b, const float* __restrict__ o,
                                                            float* __restrict__ ga, int acc_a, float* __restrict__ gb,
-                                                           int acc_b, int64_t n4) {
+                                                           int acc_b, int64_t n) {
     binary_prologue<OP>();
+    const int64_t n4 = n / 4;
     const bool need_a = (ga && da_reads_a<OP>()) || (gb && db_reads_a<OP>());
     const bool need_b = (ga && da_reads_b<OP>()) || (gb && db_reads_b<OP>()) || (gb && db_reads_out<OP>() && !o);
     const bool need_o = gb && db_reads_out<OP>() && o;
@@ -81,6 +85,15 @@ __global__ void __launch_bounds__(kBlock) bwd_flat_kernel(const float* __restric
                 st_stream(gb + e, r);
             }
         }
+    }
+    // n % 4 elements.
+    const int64_t e = n4 * 4 + threadIdx.x;
+    if (blockIdx.x == 0 && e < n) {
+        float da, db;
+        binary_grads<OP>(g[e], need_a ? a[e] : 0.f, need_b ? b[e] : 0.f, need_o ? o[e] : 0.f, need_o, ga != nullptr,
+                         gb != nullptr, da, db);
+        if (ga) ga[e] = acc_a ? ga[e] + da : da;
+        if (gb) gb[e] = acc_b ? gb[e] + db : db;
     }
 }
 
@@ -170,8 +183,8 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
     if (want_v) *reinterpret_cast<float4*>(part + (int64_t)blockIdx.y * C + c) = s;
 }
 
-// out[c] (+)= sum_k part[k, c], k in 0..K-1.  A workgroup owns S adjacent
-// columns and its threads form G = 256 / S groups: group g folds partial
+// out[o, c] (+)= sum_k part[o, k, c], k in 0..K-1.  A workgroup owns S adjacent
+// columns of one o and its threads form G = 256 / S groups: group g folds partial
 // rows k = g, g + G, g + 2G, ... (8 interleaved accumulators, combined in a
 // fixed order), and the G group sums are added in group order through LDS.
 // S is chosen so the grid has ~256 workgroups or more: with few columns
@@ -180,20 +193,23 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
 // rows per wave (13.6 us).
 template <int S>
 __global__ void __launch_bounds__(kBlock) colsum_finalize_kernel(const float* __restrict__ part, float* __restrict__ out,
-                                                                  int acc, int64_t K, int64_t C) {
+                                                                  int acc, int64_t K, int64_t C, int64_t O) {
     constexpr int G = kBlock / S;
     __shared__ float lds[G][S];
     const int cl = threadIdx.x % S, g = threadIdx.x / S;
-    for (int64_t c0 = (int64_t)blockIdx.x * S; c0 < C; c0 += (int64_t)gridDim.x * S) {
-        const int64_t c = c0 + cl;
+    const int64_t tiles = (C + S - 1) / S;
+    for (int64_t item = blockIdx.x; item < O * tiles; item += gridDim.x) {
+        const int64_t ou = item / tiles;
+        const int64_t c = (item - ou * tiles) * S + cl;
+        const float* pt = part + ou * K * C;
         float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         if (c < C) {
             int64_t k = g;
             for (; k + 7 * G < K; k += 8 * G) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) s[j] += part[(k + j * G) * C + c];
+                for (int j = 0; j < 8; ++j) s[j] += pt[(k + j * G) * C + c];
             }
-            for (int j = 0; k < K; k += G, ++j) s[j & 7] += part[k * C + c];
+            for (int j = 0; k < K; k += G, ++j) s[j & 7] += pt[k * C + c];
         }
         lds[g][cl] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
         __syncthreads();
@@ -201,21 +217,23 @@ __global__ void __launch_bounds__(kBlock) colsum_finalize_kernel(const float* __
             float t = lds[0][cl];
 #pragma unroll
             for (int gg = 1; gg < G; ++gg) t += lds[gg][cl];
-            out[c] = acc ? out[c] + t : t;
+            float* dst = out + ou * C + c;
+            *dst = acc ? *dst + t : t;
         }
         __syncthreads();
     }
 }
 
 // colsum_finalize_kernel with its column slot width chosen for C.
-int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, int64_t C, hipStream_t st) {
-    const int64_t want = (int64_t)num_cus();
-    if (C >= 64 * want)
-        launch_kernel(colsum_finalize_kernel<64>, dim3(grid_for(C, 64, 8)), dim3(kBlock), 0, st, part, out, acc, K, C);
-    else if (C >= 16 * want)
-        launch_kernel(colsum_finalize_kernel<16>, dim3(grid_for(C, 16, 8)), dim3(kBlock), 0, st, part, out, acc, K, C);
-    else
-        launch_kernel(colsum_finalize_kernel<4>, dim3(grid_for(C, 4, 8)), dim3(kBlock), 0, st, part, out, acc, K, C);
+int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, int64_t C, int64_t O, hipStream_t st) {
+    const int64_t want = (int64_t)num_cus(), cols = C * O;
+#define WM_CF(S)                                                                                             \
+    launch_kernel(colsum_finalize_kernel<S>, dim3(grid_for((C + S - 1) / S * O, 1, 8)), dim3(kBlock), 0, st, \
+                  part, out, acc, K, C, O)
+    if (cols >= 64 * want) WM_CF(64);
+    else if (cols >= 16 * want) WM_CF(16);
+    else WM_CF(4);
+#undef WM_CF
     return check_launch("wm_binary_bwd(colsum finalize)");
 }
 
@@ -458,6 +476,234 @@ __global__ void __launch_bounds__(kBlock) rowsum_finalize_kernel(const float* __
 }
 
 // ---------------------------------------------------------------------------
+// cols: F full [O,R,C], V [O,1,C] (O = 1: a row vector), any C
+// ---------------------------------------------------------------------------
+
+// A unit is a float4 (VEC: C % 4 == 0 and aligned bases) or a float.  A
+// workgroup takes `tu` adjacent units of one column tile and 256 / tu rows at
+// a time, so a short row (a ten-class bias, a 64-wide feature) still fills
+// its waves; row groups are handed out cyclically as in bwd_colsum_kernel.
+// The workgroup's row lanes are added through LDS in a fixed tree, then the
+// column sums go to the gradient (one row group) or to its partials.
+//
+// Bound by latency at small sizes (each thread keeps kColRows rows in
+// flight) and by HBM at large ones.  Before, every such layout except
+// [R, C] with C % 4 == 0 ran one thread per column over all R rows: a bias
+// gradient over [5912, 30] took 2441 us and one over [4, 27, 3616] with a
+// [4, 1, 3616] operand 16 us; rows of fewer than 1024 floats left lanes idle.
+template <int OP>
+constexpr int col_rows() { return OP == WM_POW || OP == WM_DIV ? 1 : 4; }
+
+template <int OP, bool VB, bool VEC>
+__global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restrict__ g, const float* __restrict__ F,
+                                                           const float* __restrict__ V, const float* __restrict__ o,
+                                                           float* __restrict__ gF, int accF, float* __restrict__ gV,
+                                                           int accV, float* __restrict__ part, int64_t O, int64_t R,
+                                                           int64_t C, int tu) {
+    binary_prologue<OP>();
+    constexpr int WD = VEC ? 4 : 1;
+    constexpr int UR = col_rows<OP>();
+    __shared__ float lds[kBlock][WD];
+    const bool want_v = gV != nullptr;
+    const bool gF_reads_F = VB ? da_reads_a<OP>() : db_reads_b<OP>();
+    const bool gF_reads_V = VB ? da_reads_b<OP>() : db_reads_a<OP>();
+    const bool gV_reads_F = VB ? db_reads_a<OP>() : da_reads_b<OP>();
+    const bool gV_reads_V = VB ? db_reads_b<OP>() : da_reads_a<OP>();
+    const bool want_o = VB ? (want_v && db_reads_out<OP>()) : (gF && db_reads_out<OP>());
+    const bool need_o = want_o && o;
+    const bool need_F = (gF && gF_reads_F) || (want_v && gV_reads_F) || (want_o && !o);
+    const bool need_V = (gF && gF_reads_V) || (want_v && gV_reads_V) || (want_o && !o);
+    const int rb = kBlock / tu;
+    const int tr = (int)threadIdx.x / tu, tc = (int)threadIdx.x - tr * tu;
+    const int64_t c = ((int64_t)blockIdx.x * tu + tc) * WD;
+    const bool live = tr < rb && c < C;
+    const int64_t K = gridDim.y, step = K * rb;
+    auto load = [](const float* p, float(&v)[WD]) {
+        if constexpr (VEC) {
+            const float4 q = ld_stream(p);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+            v[0] = ld_stream1(p);
+        }
+    };
+    for (int64_t ou = blockIdx.z; ou < O; ou += gridDim.z) {
+        const int64_t base = ou * R * C + c;
+        float s[WD], vv[WD];
+#pragma unroll
+        for (int j = 0; j < WD; ++j) s[j] = vv[j] = 0.f;
+        if (live && need_V) {
+#pragma unroll
+            for (int j = 0; j < WD; ++j) vv[j] = V[ou * C + c + j];
+        }
+        for (int64_t r0 = (int64_t)blockIdx.y * rb + tr; live && r0 < R; r0 += step * UR) {
+            float vg[UR][WD], vf[UR][WD], vo[UR][WD], old[UR][WD];
+#pragma unroll
+            for (int u = 0; u < UR; ++u) {
+                const int64_t r = r0 + u * step;
+                const int64_t off = base + r * C;
+                const bool in = r < R;
+#pragma unroll
+                for (int j = 0; j < WD; ++j) vg[u][j] = vf[u][j] = vo[u][j] = old[u][j] = 0.f;
+                if (in) load(g + off, vg[u]);
+                if (in && need_F) load(F + off, vf[u]);
+                if (in && need_o) load(o + off, vo[u]);
+                if (in && gF && accF) load(gF + off, old[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < UR; ++u) {
+                const int64_t r = r0 + u * step;
+                if (r >= R) break;
+                float da[WD], db[WD];
+                binary_grads_n<OP, WD>(vg[u], VB ? vf[u] : vv, VB ? vv : vf[u], vo[u], need_o,
+                                       VB ? gF != nullptr : want_v, VB ? want_v : gF != nullptr, da, db);
+                const float* dF = VB ? da : db;
+                const float* dV = VB ? db : da;
+                if (gF) {
+                    float* dst = gF + base + r * C;
+                    float d[WD];
+#pragma unroll
+                    for (int j = 0; j < WD; ++j) d[j] = accF ? dF[j] + old[u][j] : dF[j];
+                    if constexpr (VEC) st_stream(dst, make_float4(d[0], d[1], d[2], d[3]));
+                    else st_stream1(dst, d[0]);
+                }
+                if (want_v) {
+#pragma unroll
+                    for (int j = 0; j < WD; ++j) s[j] += dV[j];
+                }
+            }
+        }
+        if (!want_v) continue;
+        if (rb > 1) {
+#pragma unroll
+            for (int j = 0; j < WD; ++j) lds[threadIdx.x][j] = s[j];
+            for (int n = rb; n > 1;) {
+                const int h = (n + 1) / 2;
+                __syncthreads();
+                if (tr + h < n) {
+#pragma unroll
+                    for (int j = 0; j < WD; ++j) lds[threadIdx.x][j] += lds[threadIdx.x + h * tu][j];
+                }
+                n = h;
+            }
+#pragma unroll
+            for (int j = 0; j < WD; ++j) s[j] = lds[threadIdx.x][j];
+            __syncthreads();  // the next o writes LDS again
+        }
+        if (tr == 0 && live) {
+#pragma unroll
+            for (int j = 0; j < WD; ++j) {
+                if (K == 1) {
+                    float* dst = gV + ou * C + c + j;
+                    *dst = accV ? *dst + s[j] : s[j];
+                } else {
+                    part[(ou * K + blockIdx.y) * C + c + j] = s[j];
+                }
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// channel: F full [O,K,I], V [1,K,1] (a convolution's bias)
+// ---------------------------------------------------------------------------
+
+// Workgroup (k, chunk) walks units [chunk * per, (chunk + 1) * per) of
+// channel k's O * I / W units (W = 4: I % 4 == 0 and aligned bases), 256
+// adjacent units at a time across plane ends, so every lane has work at any
+// plane size; the position advances by the constant (256 / U planes, 256 % U
+// units) without dividing.  kChanUnits steps' loads are in flight per
+// thread.  The workgroups running at one time take the same planes of
+// neighbouring channels, which lie side by side in memory.  HBM-bound; one
+// thread per channel summing it element by element took 77.4 ms at
+// [64, 64, 56, 56].
+template <int OP>
+constexpr int chan_units() { return OP == WM_POW || OP == WM_DIV ? 1 : 4; }
+
+template <int OP, bool VB, bool VEC>
+__global__ void __launch_bounds__(kBlock) bwd_channel_kernel(
+    const float* __restrict__ g, const float* __restrict__ F, const float* __restrict__ V,
+    const float* __restrict__ o, float* __restrict__ gF, int accF, float* __restrict__ gV, int accV,
+    float* __restrict__ part, int64_t O, int64_t K, int64_t I, int64_t per) {
+    binary_prologue<OP>();
+    constexpr int WD = VEC ? 4 : 1;
+    constexpr int UR = chan_units<OP>();
+    __shared__ float lds[kBlock / 64];
+    const bool want_v = gV != nullptr;
+    const bool gF_reads_F = VB ? da_reads_a<OP>() : db_reads_b<OP>();
+    const bool gF_reads_V = VB ? da_reads_b<OP>() : db_reads_a<OP>();
+    const bool gV_reads_F = VB ? db_reads_a<OP>() : da_reads_b<OP>();
+    const bool gV_reads_V = VB ? db_reads_b<OP>() : da_reads_a<OP>();
+    const bool want_o = VB ? (want_v && db_reads_out<OP>()) : (gF && db_reads_out<OP>());
+    const bool need_o = want_o && o;
+    const bool need_F = (gF && gF_reads_F) || (want_v && gV_reads_F) || (want_o && !o);
+    const bool need_V = (gF && gF_reads_V) || (want_v && gV_reads_V) || (want_o && !o);
+    const int64_t k = blockIdx.x;
+    const int64_t U = I / WD, total = O * U;  // units per plane, per channel
+    const int64_t u0 = (int64_t)blockIdx.y * per, u1 = min(total, u0 + per);
+    const float v1 = need_V ? V[k] : 0.f;
+    float vv[WD], s[WD];
+#pragma unroll
+    for (int j = 0; j < WD; ++j) { vv[j] = v1; s[j] = 0.f; }
+    auto load = [](const float* p, float(&v)[WD]) {
+        if constexpr (VEC) {
+            const float4 q = ld_stream(p);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+            v[0] = ld_stream1(p);
+        }
+    };
+    const int64_t step_o = kBlock / U, step_i = kBlock - step_o * U;
+    int64_t u = u0 + threadIdx.x;
+    int64_t po = u / U, pi = u - po * U;  // this thread's plane and unit
+    for (; u < u1; u += kBlock * UR) {
+        int64_t off[UR];
+        float vg[UR][WD], vf[UR][WD], vo[UR][WD], old[UR][WD];
+#pragma unroll
+        for (int q = 0; q < UR; ++q) {
+            off[q] = (po * K + k) * I + pi * WD;
+            const bool in = u + q * kBlock < u1;
+#pragma unroll
+            for (int j = 0; j < WD; ++j) vg[q][j] = vf[q][j] = vo[q][j] = old[q][j] = 0.f;
+            if (in) load(g + off[q], vg[q]);
+            if (in && need_F) load(F + off[q], vf[q]);
+            if (in && need_o) load(o + off[q], vo[q]);
+            if (in && gF && accF) load(gF + off[q], old[q]);
+            po += step_o;
+            pi += step_i;
+            if (pi >= U) { pi -= U; ++po; }
+        }
+#pragma unroll
+        for (int q = 0; q < UR; ++q) {
+            if (u + q * kBlock >= u1) break;
+            float da[WD], db[WD];
+            binary_grads_n<OP, WD>(vg[q], VB ? vf[q] : vv, VB ? vv : vf[q], vo[q], need_o,
+                                   VB ? gF != nullptr : want_v, VB ? want_v : gF != nullptr, da, db);
+            const float* dF = VB ? da : db;
+            const float* dV = VB ? db : da;
+            if (gF) {
+                float d[WD];
+#pragma unroll
+                for (int j = 0; j < WD; ++j) d[j] = accF ? dF[j] + old[q][j] : dF[j];
+                if constexpr (VEC) st_stream(gF + off[q], make_float4(d[0], d[1], d[2], d[3]));
+                else st_stream1(gF + off[q], d[0]);
+            }
+            if (want_v) {
+#pragma unroll
+                for (int j = 0; j < WD; ++j) s[j] += dV[j];
+            }
+        }
+    }
+    if (!want_v) return;
+    float t = s[0];
+    if constexpr (VEC) t = (s[0] + s[1]) + (s[2] + s[3]);
+    t = block_sum<kBlock>(t, lds);
+    if (threadIdx.x == 0) {
+        if (gridDim.y == 1) gV[k] = accV ? gV[k] + t : t;
+        else part[k * gridDim.y + blockIdx.y] = t;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // generic: one thread per operand element
 // ---------------------------------------------------------------------------
 
@@ -519,6 +765,64 @@ __global__ void __launch_bounds__(kBlock) bwd_generic_kernel(const float* __rest
 // Host dispatch
 // ---------------------------------------------------------------------------
 
+// [O, R, C] with V [O, 1, C].  64 adjacent units per row and workgroup (a
+// contiguous 1 KB of float4s), fewer when a row is shorter, so small R still
+// spreads over the row lanes; row groups until ~1024 workgroups run.  A group
+// of at most 4 steps of a workgroup is not split: its steps cost less than
+// the ~4 us of the second dispatch that adds the groups' partials.
+template <int OP>
+int launch_cols(bool vb, bool vec, const float* g, const float* F, const float* V, const float* o, float* gF, int accF,
+                float* gV, int accV, int64_t O, int64_t R, int64_t C) {
+    hipStream_t st = stream();
+    const int64_t units = vec ? C / 4 : C;
+    const int tu = (int)std::min<int64_t>(units, 64);
+    const int64_t tiles = (units + tu - 1) / tu;
+    const int64_t steps = (R + (int64_t)(kBlock / tu) * col_rows<OP>() - 1) / ((int64_t)(kBlock / tu) * col_rows<OP>());
+    int64_t K = 1;
+    if (steps > 4 && tiles * O < 1024) K = std::min<int64_t>(steps, (1024 + tiles * O - 1) / (tiles * O));
+    Workspace ws(gV && K > 1 ? (size_t)(O * K * C) * sizeof(float) : 0);
+    if (gV && K > 1 && !ws.p) return set_error(WM_ERR_NOMEM, "wm_binary_bwd: workspace");
+    const dim3 grid((unsigned)tiles, (unsigned)K, (unsigned)std::min<int64_t>(O, 65535));
+#define WM_BC(VBv, VECv)                                                                                          \
+    launch_kernel((bwd_cols_kernel<OP, VBv, VECv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV, accV,    \
+                  ws.as<float>(), O, R, C, tu)
+    if (vb) { if (vec) WM_BC(true, true); else WM_BC(true, false); }
+    else { if (vec) WM_BC(false, true); else WM_BC(false, false); }
+#undef WM_BC
+    WM_TRY(check_launch("wm_binary_bwd(cols)"));
+    if (gV && K > 1) return launch_colsum_finalize(ws.as<float>(), gV, accV, K, C, O, st);
+    return WM_OK;
+}
+
+// [O, K, I] with V [1, K, 1]: chunks of at least 4 steps of a workgroup until
+// ~8 workgroups per CU run.
+template <int OP>
+int launch_channel(bool vb, bool vec, const float* g, const float* F, const float* V, const float* o, float* gF,
+                   int accF, float* gV, int accV, int64_t O, int64_t K, int64_t I) {
+    hipStream_t st = stream();
+    const int64_t total = O * (vec ? I / 4 : I), step = kBlock * chan_units<OP>();
+    const int64_t want = std::max<int64_t>(1, (int64_t)num_cus() * 8 / K);
+    const int64_t chunks0 = std::min<int64_t>(std::min<int64_t>(want, (total + 4 * step - 1) / (4 * step)), 65535);
+    const int64_t per = ((total + chunks0 - 1) / chunks0 + step - 1) / step * step;
+    const int64_t chunks = (total + per - 1) / per;
+    Workspace ws(gV && chunks > 1 ? (size_t)(K * chunks) * sizeof(float) : 0);
+    if (gV && chunks > 1 && !ws.p) return set_error(WM_ERR_NOMEM, "wm_binary_bwd: workspace");
+    const dim3 grid((unsigned)K, (unsigned)chunks);
+#define WM_CH(VBv, VECv)                                                                                          \
+    launch_kernel((bwd_channel_kernel<OP, VBv, VECv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV, accV, \
+                  ws.as<float>(), O, K, I, per)
+    if (vb) { if (vec) WM_CH(true, true); else WM_CH(true, false); }
+    else { if (vec) WM_CH(false, true); else WM_CH(false, false); }
+#undef WM_CH
+    WM_TRY(check_launch("wm_binary_bwd(channel)"));
+    if (gV && chunks > 1) {
+        launch_kernel(rowsum_finalize_kernel, dim3(grid_for(K, 1, 8)), dim3(kBlock), 0, st, ws.as<float>(), gV, accV,
+                      K, chunks);
+        return check_launch("wm_binary_bwd(channel finalize)");
+    }
+    return WM_OK;
+}
+
 template <int OP>
 int launch_binary_bwd(const float* g, const float* a, const float* b, const float* o, float* ga, int acc_a, float* gb,
                       int acc_b, int nd, const int64_t* size, const int64_t* sa, const int64_t* sb, int64_t numel,
@@ -538,11 +842,34 @@ int launch_binary_bwd(const float* g, const float* a, const float* b, const floa
 
     // flat
     if (a_full && b_full) {
-        if (numel % 4 == 0 && aligned) {
-            int64_t n4 = numel / 4;
-            launch_kernel(bwd_flat_kernel<OP>, dim3(grid_for(n4, kBlock * kSlotsFlat, 1 << 12)), dim3(kBlock), 0, st, g, a, b, o,
-                               ga, acc_a, gb, acc_b, n4);
+        if (aligned) {
+            launch_kernel(bwd_flat_kernel<OP>, dim3(grid_for(numel / 4, kBlock * kSlotsFlat, 1 << 12)), dim3(kBlock),
+                          0, st, g, a, b, o, ga, acc_a, gb, acc_b, numel);
             return check_launch("wm_binary_bwd(flat)");
+        }
+    }
+
+    // One full operand, the other repeated along one run of dims: the rows of
+    // [O, R, C] (a row vector when O = 1), or the outer and inner dims of
+    // [O, K, I] (a channel vector).
+    if (a_full != b_full && (nd == 2 || nd == 3)) {
+        const bool vb = a_full;
+        const int64_t* sv = vb ? sb : sa;
+        const float* F = vb ? a : b;
+        const float* V = vb ? b : a;
+        float* gF = vb ? ga : gb;
+        float* gV = vb ? gb : ga;
+        const int accF = vb ? acc_a : acc_b, accV = vb ? acc_b : acc_a;
+        const int64_t C = size[nd - 1];
+        const bool vec = C % 4 == 0 && aligned;
+        if (sv[nd - 1] == 1 && sv[nd - 2] == 0) {
+            const int64_t O = nd == 3 ? size[0] : 1, R = size[nd - 2];
+            // bwd_colsum_kernel keeps the wide aligned [R, C] it was shaped
+            // for (one row per step, 1024-column tiles).
+            if (!(O == 1 && vec && C >= kBlock * 4))
+                return launch_cols<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, O, R, C);
+        } else if (nd == 3 && sv[0] == 0 && sv[1] == 1 && sv[2] == 0) {
+            return launch_channel<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, size[0], size[1], C);
         }
     }
 
@@ -559,7 +886,7 @@ int launch_binary_bwd(const float* g, const float* a, const float* b, const floa
         const int accF = vb ? acc_a : acc_b, accV = vb ? acc_b : acc_a;
         const bool rowvec = nd == 2 && sv[0] == 0 && sv[1] == 1;
         const bool colvec = (nd == 2 && sv[0] == 1 && sv[1] == 0) || (nd == 1 && sv[0] == 0);
-        if (rowvec && C % 4 == 0 && aligned) {
+        if (rowvec && C % 4 == 0 && C >= kBlock * 4 && aligned) {
             const int64_t col_tiles = (C + kBlock * 4 - 1) / (kBlock * 4);
             // ~1024 workgroups (4 per CU), each group of at least 4 rows (a
             // thread walks its group's rows one at a time, so a small R needs
@@ -579,7 +906,7 @@ int launch_binary_bwd(const float* g, const float* a, const float* b, const floa
                                    ws.as<float>(), R, C);
             WM_TRY(check_launch("wm_binary_bwd(colsum)"));
             if (gV) {
-                WM_TRY(launch_colsum_finalize(ws.as<float>(), gV, accV, K, C, st));
+                WM_TRY(launch_colsum_finalize(ws.as<float>(), gV, accV, K, C, 1, st));
             }
             return WM_OK;
         }
