@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from tests.gpu_helpers import binary_bwd, binary_fwd, rng_normal, rng_uniform
+from gpu_helpers import binary_bwd, binary_fwd, gemm, rng_normal, rng_uniform
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-5
@@ -52,3 +52,43 @@ def test_broadcast_backward_edges(wm, op, full, vec):
             assert ok, f"grad a off by {w:.3g}x tolerance (swap {swap}, accumulate {acc})"
             ok, w = oracle.close_scaled(gb, rb + zb, tb + np.abs(zb), RTOL)
             assert ok, f"grad b off by {w:.3g}x tolerance (swap {swap}, accumulate {acc})"
+
+
+# One size per form of the small-tile product (16- and 32-wide tiles with k
+# over 4 or 16 waves, 64-wide tiles) and its edges: a partial step only, one
+# full step and a rest, fewer steps than waves, rows past a tile, odd leading
+# dimensions, more problems than one.
+SMALL_PRODUCTS = [(1, 1, 1, 1), (3, 17, 33, 5), (16, 16, 31, 1), (65, 128, 130, 1), (16, 512, 333, 1), (1, 70, 4100, 1),
+                  (300, 10, 768, 1), (33, 47, 8200, 1), (40, 3000, 65, 1), (700, 900, 30, 1), (1500, 1201, 97, 1),
+                  (2, 64, 333, 24)]
+
+
+@pytest.mark.parametrize("m,n,k,batch", SMALL_PRODUCTS)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_small_products(wm, m, n, k, batch, ta, tb):
+    """alpha, accumulation and bias, leading dimensions 1 and 3 past a row
+    (NaN there), against float64 within 1e-5 of the sum of |terms|."""
+    r = np.random.default_rng(seed_of(m, n, k, ta, tb))
+    a, b = r.standard_normal((batch, m, k), np.float32), r.standard_normal((batch, k, n), np.float32)
+    lda, ldb, ldc = (m if ta else k) + 1, (k if tb else n) + 3, n + 1
+
+    def stored(x, trans, ld):
+        s = x.transpose(0, 2, 1) if trans else x
+        buf = np.full(s.shape[:2] + (ld,), np.nan, np.float32)
+        buf[..., :s.shape[2]] = s
+        return buf
+
+    sa, sb = stored(a, ta, lda), stored(b, tb, ldb)
+    c0 = r.standard_normal((batch, m, ldc), np.float32)
+    bias = r.standard_normal(n, np.float32)
+    st = (sa[0].size, 0, sb[0].size, 0, c0[0].size, 0)
+    ref = np.matmul(a.astype(np.float64), b)
+    scale = np.matmul(np.abs(a).astype(np.float64), np.abs(b))
+    for acc, bi in ((0, None), (1, None), (0, bias), (1, bias)):
+        got = gemm(ta, tb, m, n, k, 0.5, sa.ravel(), lda, sb.ravel(), ldb, c0.ravel(), ldc, acc, bi, batch, 1, st)
+        got = got.reshape(c0.shape)
+        add = (c0[..., :n] if acc else 0.0) + (bias if bi is not None else 0.0)
+        size = (np.abs(c0[..., :n]) if acc else 0.0) + (np.abs(bias) if bi is not None else 0.0)
+        ok, w = oracle.close_scaled(got[..., :n], 0.5 * ref + add, 0.5 * scale + size, RTOL)
+        assert ok, f"{w:.3g}x tolerance"
+        assert np.array_equal(got[..., n:], c0[..., n:])  # past the rows: untouched

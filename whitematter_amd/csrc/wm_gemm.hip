@@ -51,6 +51,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <cmath>
 #include <mutex>
 
 namespace wm {
@@ -991,6 +992,194 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restr
     }
 }
 
+// ---- few or small tiles: operands straight into fragments ------------------
+//
+// A product with few 128 x 128 tiles leaves most of the chip idle on the
+// kernels above: a 64 x 128 output is one workgroup walking all of k.  Here a
+// workgroup computes a small tile, and its WK waves split k among themselves:
+// wave w takes k steps w, w + WK, ..., and the waves' accumulators are added
+// through LDS in wave order.  Each wave loads its MFMA fragments from global
+// memory straight into registers, two steps ahead: a k-contiguous operand as
+// 16-byte loads (at 4-byte alignment, so any leading dimension takes the same
+// path), a row-contiguous one as dwords along the row.  The operands of such
+// products come from the caches, so LDS staging would only add barriers.
+//   BLK = 16: v_mfma_f32_16x16x4_f32, lane quarter q takes k 8q .. 8q + 7 of
+//             a 32-k step;
+//   BLK = 32: v_mfma_f32_32x32x2_f32, lane half h takes k 8h .. 8h + 7 of a
+//             16-k step.
+// WR x WC waves (WK = 1 then) tile a (WR BLK) x (WC BLK) output each for
+// themselves; their repeated reads of a row or column panel hit the L1.
+// Rows and columns past the edge read the last valid one (their results are
+// not stored); only the last, partial k step is read element by element.
+//
+// Bound by the latency of a wave's chain of k steps at small sizes and by the
+// caches' bandwidth (43-70 TFLOP/s) at large ones, where the 128-row kernels
+// and the library take over (choose_small).  (64, 784) x (784, 128) took 83 us
+// on one 128-row tile and takes 5.5; a Linear of that size, forward and
+// backward, 127.8 -> 20.3 us.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int BLK>
+struct SmallAcc;
+template <>
+struct SmallAcc<16> {
+    using T = f32x4;
+    static constexpr int Q = 4;
+    __device__ __forceinline__ static T mma(float a, float b, T c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int row(int q, int lane) { return 4 * (lane >> 4) + q; }
+};
+template <>
+struct SmallAcc<32> {
+    using T = f32x16;
+    static constexpr int Q = 16;
+    __device__ __forceinline__ static T mma(float a, float b, T c) {
+        return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ static int row(int q, int lane) { return 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3); }
+};
+
+// A lane's 8 k values of one operand in one step.  KC: element (row, k) at
+// base[row * ld + k], else at base[k * ld + row]; `lane_bytes` is the lane's
+// byte offset from its block's first row at the step's first k.
+template <bool KC>
+struct SmallFrag {
+    float v[8];
+    __device__ __forceinline__ static uint32_t lane_bytes(int row, int sub, int64_t ld) {
+        return 4u * (KC ? (uint32_t)row * (uint32_t)ld + 8u * (uint32_t)sub : 8u * (uint32_t)sub * (uint32_t)ld + (uint32_t)row);
+    }
+    // `p`: the block's first row at the step's first k (wave-uniform).
+    __device__ __forceinline__ void load(const float* p, uint32_t off, int64_t ld) {
+        if constexpr (KC) {
+            const char* b = reinterpret_cast<const char*>(p);
+            const f32x4u x = *reinterpret_cast<const f32x4u*>(b + off);
+            const f32x4u y = *reinterpret_cast<const f32x4u*>(b + off + 16);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { v[j] = x[j]; v[4 + j] = y[j]; }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(p + j * ld) + off);
+        }
+    }
+    // The partial step: the lane's k values are k .. k + 7 of `left` valid
+    // ones from the step's first.
+    __device__ __forceinline__ void load_tail(const float* p, uint32_t off, int64_t ld, int k, int left) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[j] = 0.0f;
+            if (k + j < left)
+                v[j] = *reinterpret_cast<const float*>(
+                    reinterpret_cast<const char*>(p + (KC ? (int64_t)j : j * ld)) + off);
+        }
+    }
+};
+
+template <bool TA, bool TB, int BLK, int WR, int WC, int WK>
+__global__ void __launch_bounds__(64 * WR * WC * WK) gemm_small_kernel(GemmParams P) {
+    static_assert(WK == 1 || (WR == 1 && WC == 1), "waves split k or the tile");
+    using Acc = SmallAcc<BLK>;
+    using FA = SmallFrag<!TA>;
+    using FB = SmallFrag<TB>;
+    constexpr int SUBS = 64 / BLK;   // lane groups along k
+    constexpr int STEP = 8 * SUBS;   // k per step
+    constexpr int NT = 64 * WR * WC * WK;
+    __shared__ float red[WK > 1 ? WK * BLK * BLK : 1];
+
+    const int ntiles = P.tiles_m * P.tiles_n;
+    int t = (int)blockIdx.x;
+    if ((ntiles & 7) == 0) t = (t & 7) * (ntiles >> 3) + (t >> 3);
+    int tm, tn;
+    tile_of(t, P.tiles_m, P.tiles_n, tm, tn);
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wk = WK > 1 ? wave : 0;
+    const int wr = WK > 1 ? 0 : wave / WC, wc = WK > 1 ? 0 : wave % WC;
+    const int64_t m0 = (int64_t)tm * (WR * BLK) + wr * BLK, n0 = (int64_t)tn * (WC * BLK) + wc * BLK;
+    if (WK == 1 && (m0 >= P.m || n0 >= P.n)) return;  // no barrier below when WK == 1
+    const int r = lane & (BLK - 1), sub = lane / BLK;
+    const uint32_t aoff = FA::lane_bytes((int)min((int64_t)r, P.m - 1 - m0), sub, P.lda);
+    const uint32_t boff = FB::lane_bytes((int)min((int64_t)r, P.n - 1 - n0), sub, P.ldb);
+
+    const int64_t nprob = P.batch * P.kslices;
+    for (int64_t p = blockIdx.y; p < nprob; p += gridDim.y) {
+        const int64_t pb = p / P.kslices, ks = p - pb * P.kslices;
+        const int64_t po = pb / P.batch_inner, pi = pb - po * P.batch_inner;
+        const int64_t kb = ks * P.ksplit;
+        const int64_t kdim = min(P.ksplit, P.k - kb);
+        const float* A = P.a + po * P.sa0 + pi * P.sa1 + (TA ? kb * P.lda + m0 : m0 * P.lda + kb);
+        const float* B = P.b + po * P.sb0 + pi * P.sb1 + (TB ? n0 * P.ldb + kb : kb * P.ldb + n0);
+        float* C = P.c + po * P.sc0 + pi * P.sc1 + ks * P.sck;
+        const int64_t as = TA ? STEP * P.lda : STEP, bs = TB ? STEP : STEP * P.ldb;  // floats per step
+
+        typename Acc::T acc;
+#pragma unroll
+        for (int q = 0; q < Acc::Q; ++q) acc[q] = 0.0f;
+        auto mma = [&](const FA& a, const FB& b) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = Acc::mma(a.v[j], b.v[j], acc);
+        };
+        const int nfull = (int)(kdim / STEP);
+        if (wk < nfull) {
+            // Steps past the wave's last load that one again (never used), so
+            // the loop has no branch around its loads.
+            const int last = nfull - 1 - (nfull - 1 - wk) % WK;
+            FA a0, a1, a2;
+            FB b0, b1, b2;
+            a0.load(A + wk * as, aoff, P.lda);
+            b0.load(B + wk * bs, boff, P.ldb);
+            const int s1 = min(wk + WK, last);
+            a1.load(A + s1 * as, aoff, P.lda);
+            b1.load(B + s1 * bs, boff, P.ldb);
+            for (int s = wk; s < nfull; s += WK) {
+                const int s2 = min(s + 2 * WK, last);
+                a2.load(A + s2 * as, aoff, P.lda);
+                b2.load(B + s2 * bs, boff, P.ldb);
+                mma(a0, b0);
+                a0 = a1;
+                b0 = b1;
+                a1 = a2;
+                b1 = b2;
+            }
+        }
+        const int left = (int)(kdim - (int64_t)nfull * STEP);
+        if (left > 0 && wk == nfull % WK) {
+            FA a;
+            FB b;
+            a.load_tail(A + nfull * as, aoff, P.lda, 8 * sub, left);
+            b.load_tail(B + nfull * bs, boff, P.ldb, 8 * sub, left);
+            mma(a, b);
+        }
+
+        const float alpha = P.alpha;
+        auto put = [&](int row, int col, float x) {
+            if (m0 + row >= P.m || n0 + col >= P.n) return;
+            float* dst = C + (m0 + row) * P.ldc + n0 + col;
+            x = alpha * x;
+            if (P.accumulate) x = *dst + x;
+            if (P.bias) x = x + P.bias[n0 + col];
+            *dst = x;
+        };
+        if constexpr (WK == 1) {
+#pragma unroll
+            for (int q = 0; q < Acc::Q; ++q) put(Acc::row(q, lane), r, acc[q]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < Acc::Q; ++q) red[wk * BLK * BLK + q * 64 + lane] = acc[q];
+            __syncthreads();
+            for (int e = (int)threadIdx.x; e < BLK * BLK; e += NT) {
+                float x = red[e];
+#pragma unroll
+                for (int w = 1; w < WK; ++w) x += red[w * BLK * BLK + e];
+                put(Acc::row(e >> 6, e & 63), (e & 63) & (BLK - 1), x);
+            }
+            __syncthreads();  // the next problem writes the sums again
+        }
+    }
+}
+
 // Slices per problem for a launch of `work` workgroups (tiles x problems)
 // over a k extent of k: a launch that leaves most of the chip idle (fewer
 // workgroups than CUs; two fit on each) and has a long k is cut into k
@@ -1056,24 +1245,28 @@ __global__ void __launch_bounds__(256) bias_rows_kernel(float* __restrict__ c, i
 
 bool fits_int(int64_t v) { return v >= 0 && v <= INT_MAX; }
 
-// The library route for P, or 1 when it does not take P (the caller then
-// launches gemm_kernel); WM_OK or an error status when it ran.
-int try_library(bool ta, bool tb, const GemmParams& P) {
-    if (!g_library.load(std::memory_order_relaxed) || P.kslices > 1) return 1;
-    if (P.m < 128 || P.n < 128) return 1;
-    if (P.bias && P.accumulate) return 1;
+// Whether the library's kernels are the ones for P (see above).
+bool library_takes(bool ta, bool tb, const GemmParams& P) {
+    if (P.m < 128 || P.n < 128) return false;
+    if (P.bias && P.accumulate) return false;
     if (P.batch != 1) {
         // One-level batches of untransposed small-k products (bmm's forward);
         // their gradients and the attention's two-level per-head products
         // measured slower on the library and stay on gemm_kernel.
-        if (P.batch_inner != 1 || ta || tb || P.k > 256 || P.bias) return 1;
-        if (P.sc0 < P.m * P.ldc) return 1;  // problems sharing output rows stay on gemm_kernel
+        if (P.batch_inner != 1 || ta || tb || P.k > 256 || P.bias) return false;
+        if (P.sc0 < P.m * P.ldc) return false;  // problems sharing output rows stay on gemm_kernel
     } else if (P.k < 256) {
-        return 1;
+        return false;
     }
-    if (!fits_int(P.m) || !fits_int(P.n) || !fits_int(P.k) || !fits_int(P.lda) || !fits_int(P.ldb) ||
-        !fits_int(P.ldc) || !fits_int(P.batch))
-        return 1;
+    return fits_int(P.m) && fits_int(P.n) && fits_int(P.k) && fits_int(P.lda) && fits_int(P.ldb) &&
+           fits_int(P.ldc) && fits_int(P.batch);
+}
+
+// The library route for P, or 1 when it does not take P (the caller then
+// launches gemm_kernel); WM_OK or an error status when it ran.
+int try_library(bool ta, bool tb, const GemmParams& P) {
+    if (!g_library.load(std::memory_order_relaxed) || P.kslices > 1) return 1;
+    if (!library_takes(ta, tb, P)) return 1;
     const int64_t sc = 0;
     Blas& B = blas();
     std::lock_guard<std::mutex> lk(B.mu);
@@ -1172,6 +1365,77 @@ int launch_dma32(GemmParams P, int64_t tiles) {
     return check_launch("wm_gemm(dma32)");
 }
 
+// Which kernel takes a product that the library does not: an estimate of each
+// form's time, in us, from how a grid of such tiles ran on MI355X (m, n, k
+// from 1 to 8192, all transposes): a start, then the longer of one wave's
+// chain of k steps and the chip's rate over all tiles.
+//   16 x 16, k over 4 or 16 waves   2.8 + max(0.50 S, T (WK 0.00055 + steps 0.00038))
+//   32 x 32, k over 4 waves         3.3 + max(0.45 S, T (0.0022 + steps 0.00056))
+//   64 x 64, a wave per quarter     4.0 + max(0.41 S, T (0.0022 + steps 0.0018))
+//   128-row tiles                   5.0 + max(2.5 nk (1.5 from LDS), T nk 0.0105), 5 more when k is split
+// (S: k steps of one wave, T: tiles of all problems, nk: 32-k stages; half
+// the rate's term for 64-wide tiles.)  Measured on both sides, small / 128-row:
+//   (64, 128, 784) 5.5 / 83, (784, 128, 64)^T 3.5 / 12.8, (16, 512, 512) 5.2 / 50,
+//   (4096, 10, 768) 6.7 / 62, (32, 32, 8192) 20 / 30, (5912, 1392, 30) 18 / 34,
+//   (3072, 768, 128) 16.3 / 15.5, (2624, 2576, 221) 51 / 60 us.
+enum SmallForm { kNoSmall, kSmall16x4, kSmall16x16, kSmall32x4, kSmall64 };
+
+double big_us(const GemmParams& P, bool lds_dma, bool narrow, bool vec, int64_t work) {
+    const int64_t ks = lds_dma ? 1 : choose_kslices(work, P.k);
+    const double nk = std::ceil((double)P.k / (double)ks / kBK);
+    const double stage = (vec ? 0.0105 : 0.016) * (narrow ? 0.5 : 1.0);
+    return 5.0 + std::max((lds_dma ? 1.5 : 2.5) * nk, (double)work * ks * nk * stage) + (ks > 1 ? 5.0 : 0.0);
+}
+
+SmallForm choose_small(const GemmParams& P, double limit_us) {
+    // 32-bit lane offsets: at most 32 rows of the leading dimension in bytes.
+    if (P.lda > (1 << 23) || P.ldb > (1 << 23) || P.k > INT_MAX) return kNoSmall;
+    auto tiles = [&](int64_t b) { return (double)((P.m + b - 1) / b) * (double)((P.n + b - 1) / b); };
+    if (tiles(16) > (double)INT_MAX) return kNoSmall;
+    SmallForm best = kNoSmall;
+    auto consider = [&](SmallForm f, int64_t blk, double start, double per_step, double per_tile, double rate,
+                        int64_t kstep, int64_t wk) {
+        const double steps = std::ceil((double)P.k / (double)kstep);
+        const double us = start + std::max(per_step * std::ceil(steps / (double)wk),
+                                           tiles(blk) * (double)P.batch * (per_tile + steps * rate));
+        if (us < limit_us) {
+            limit_us = us;
+            best = f;
+        }
+    };
+    consider(kSmall16x4, 16, 2.8, 0.50, 0.0022, 0.00038, 32, 4);
+    consider(kSmall16x16, 16, 2.8, 0.50, 0.0088, 0.00038, 32, 16);
+    consider(kSmall32x4, 32, 3.3, 0.45, 0.0022, 0.00056, 16, 4);
+    consider(kSmall64, 64, 4.0, 0.41, 0.0022, 0.0018, 16, 1);
+    return best;
+}
+
+template <int BLK, int WR, int WC, int WK>
+int launch_small_form(bool ta, bool tb, GemmParams P) {
+    P.tiles_m = (int)((P.m + WR * BLK - 1) / (WR * BLK));
+    P.tiles_n = (int)((P.n + WC * BLK - 1) / (WC * BLK));
+    P.kslices = 1;
+    P.ksplit = P.k;
+    P.sck = 0;
+    const dim3 grid((unsigned)(P.tiles_m * P.tiles_n), (unsigned)std::min<int64_t>(P.batch, 65535));
+    const dim3 block(64 * WR * WC * WK);
+    hipStream_t st = stream();
+    if (!ta && !tb) launch_kernel((gemm_small_kernel<false, false, BLK, WR, WC, WK>), grid, block, 0, st, P);
+    else if (!ta && tb) launch_kernel((gemm_small_kernel<false, true, BLK, WR, WC, WK>), grid, block, 0, st, P);
+    else if (ta && !tb) launch_kernel((gemm_small_kernel<true, false, BLK, WR, WC, WK>), grid, block, 0, st, P);
+    else launch_kernel((gemm_small_kernel<true, true, BLK, WR, WC, WK>), grid, block, 0, st, P);
+    return check_launch("wm_gemm(small)");
+}
+
+int launch_small(SmallForm f, bool ta, bool tb, const GemmParams& P) {
+    switch (f) {
+        case kSmall16x4: return launch_small_form<16, 1, 1, 4>(ta, tb, P);
+        case kSmall16x16: return launch_small_form<16, 1, 1, 16>(ta, tb, P);
+        case kSmall32x4: return launch_small_form<32, 1, 1, 4>(ta, tb, P);
+        default: return launch_small_form<32, 2, 2, 1>(ta, tb, P);
+    }
+}
+
 int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
     GemmParams P = P0;
     // 64-wide column tiles for narrow products (attention's per-head products
@@ -1189,15 +1453,25 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
     hipStream_t s = stream();
     P.kslices = 1;
     P.group = 1;
-    // Batched products that fit gemm_dma_kernel run there (faster than the
-    // library's strided-batched kernels on them); plain ones keep the library
-    // unless its route is switched off.
-    if (dma_fits(vec, P, tm * tn) && (P.batch > 1 || !g_library.load(std::memory_order_relaxed))) {
+    // The library keeps its plain large products, and its batched ones that
+    // fill the chip; the estimates above choose between small tiles, the
+    // direct-to-LDS kernels where a batch fits them, and gemm_kernel for the
+    // rest.  With the library route off every product runs on the 128-row
+    // kernels.
+    const bool routed = g_library.load(std::memory_order_relaxed) != 0;
+    const int64_t work = tm * tn * P.batch;
+    const bool dma = dma_fits(vec, P, tm * tn) && (P.batch > 1 || !routed);
+    const bool dma32 = narrow && dma32_fits(ta, tb, vec, P, tm * tn) && (P.batch > 1 || !routed);
+    const bool lib_first = library_takes(ta, tb, P) && (P.batch == 1 || work >= num_cus());
+    if (routed && P.k > 0 && !lib_first) {
+        const SmallForm f = choose_small(P, big_us(P, dma || dma32, narrow, vec, work));
+        if (f != kNoSmall) return launch_small(f, ta, tb, P);
+    }
+    if (dma) {
         const int r = launch_dma(ta, tb, P, tm * tn);
         if (r != 1) return r;
     }
-    if (narrow && dma32_fits(ta, tb, vec, P, tm * tn) &&
-        (P.batch > 1 || !g_library.load(std::memory_order_relaxed))) {
+    if (dma32) {
         const int r = launch_dma32(P, tm * tn);
         if (r != 1) return r;
     }
