@@ -1,12 +1,13 @@
 """Sizes at the edges of the kernels' tiles: short, odd and unaligned rows,
 small planes, one-row and many-row reductions."""
+import ctypes as C
 import zlib
 
 import numpy as np
 import pytest
 
 import oracle
-from gpu_helpers import binary_bwd, binary_fwd, gemm, rng_normal, rng_uniform
+from gpu_helpers import _offset_dev, binary_bwd, binary_fwd, gemm, rng_normal, rng_uniform
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-5
@@ -92,3 +93,39 @@ def test_small_products(wm, m, n, k, batch, ta, tb):
         ok, w = oracle.close_scaled(got[..., :n], 0.5 * ref + add, 0.5 * scale + size, RTOL)
         assert ok, f"{w:.3g}x tolerance"
         assert np.array_equal(got[..., n:], c0[..., n:])  # past the rows: untouched
+
+
+@pytest.mark.parametrize("offset", [0, 1, 2])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (7, 4), (600, 13), (3, 127), (300, 255), (5, 1023), (4, 1024),
+                                       (3, 1025), (2, 4099), (3, 32772), (2, 33001)])
+def test_cross_entropy_rows_at_any_alignment(wm, rows, cols, offset):
+    """Logits and gradient starting `offset` floats past a 16-byte boundary:
+    loss and gradient (written, then accumulated) within 1e-5 of the fp64
+    oracle's scale, and nothing written before or after the gradient."""
+    s = seed_of("ce", rows, cols)
+    x = rng_normal((rows, cols), s, 3.0)
+    x[0, cols // 2] = 40.0
+    if cols > 4:
+        x[-1, :cols // 3] = -np.inf
+    lab = (np.arange(rows) * 7 + cols - 1) % cols
+    lab[-1] = cols - 1  # a -inf label entry would make the loss infinite, with nothing left to compare
+    dx, px = _offset_dev(x, offset)
+    dl, dg = wm.DeviceArray.from_host(lab.astype(np.float32)), wm.DeviceArray.from_host(np.float32([0.75]))
+    stats, loss = wm.DeviceArray((rows, wm.CE_STATS)), wm.DeviceArray((1,))
+    wm.call("wm_cross_entropy_fwd", px, dl.vp, rows, cols, stats.vp, loss.vp)
+    ref = oracle.get("f64").cross_entropy(x, lab.astype(np.float32))
+    assert abs(loss.to_host()[0] - ref) <= RTOL * max(abs(ref), 1.0)
+    buf = rng_normal((offset + rows * cols + 8,), s + 1)
+    gx = wm.DeviceArray.from_host(buf)
+    pg = C.c_void_p(gx.ptr + 4 * offset)
+    r64 = oracle.get("f64").cross_entropy_bwd(x, lab.astype(np.float32), 0.75)
+    scale = oracle.get("abs").cross_entropy_bwd(x, lab.astype(np.float32), 0.75)
+    for acc in (1, 0):
+        wm.call("wm_cross_entropy_bwd", px, dl.vp, stats.vp, dg.vp, pg, acc, rows, cols)
+        got = gx.to_host()
+        g = got[offset:offset + rows * cols].reshape(rows, cols)
+        g0 = buf[offset:offset + rows * cols].reshape(rows, cols) if acc else np.zeros((rows, cols), np.float32)
+        ok, w = oracle.close_scaled(g, r64 + g0, scale + np.abs(g0), RTOL, 1e-30)
+        assert ok, f"{w:.3g}x tolerance (accumulate {acc})"
+        assert np.array_equal(got[:offset], buf[:offset])
+        assert np.array_equal(got[offset + rows * cols:], buf[offset + rows * cols:])

@@ -105,6 +105,16 @@ __device__ __forceinline__ void st_stream(float* p, float4 v) {
     __builtin_nontemporal_store(w, reinterpret_cast<wm_v4f*>(p));
 }
 
+// A 128-bit streaming load at 4-byte alignment (the hardware takes it): rows
+// whose length is not a multiple of 4 start anywhere, and a wave's load is
+// still one contiguous span.
+typedef float wm_v4fu __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ float4 ld_unaligned(const float* p) {
+    wm_v4fu v = __builtin_nontemporal_load(reinterpret_cast<const wm_v4fu*>(p));
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+
 __device__ __forceinline__ float ld_stream1(const float* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_stream1(float* p, float v) { __builtin_nontemporal_store(v, p); }
 

@@ -117,26 +117,45 @@ __global__ void __launch_bounds__(NT) head_fwd_kernel(const float* __restrict__ 
 }
 
 // Online single pass for long rows: each thread keeps a running max m_t and
-// the sum s_t of exp(x - m_t) over its elements, rescaling s_t when m_t
-// grows; the workgroup then combines them as row_max_sum does.  -inf
-// elements contribute nothing (exp(-inf) = 0); an element equal to a +inf
-// max contributes exp(inf - inf) = NaN, as in the reference.
+// the sum s_t of exp(x - m_t) over its elements, rescaling s_t when a step's
+// max exceeds m_t; the workgroup then combines them as row_max_sum does.
+// -inf elements contribute nothing (exp(-inf) = 0); an element equal to a
+// +inf max contributes exp(inf - inf) = NaN, as in the reference.  Four
+// 128-bit loads per thread and step at the row's own alignment: 144 -> 77 us at
+// [2048, 50257] against one float per thread and step.
 template <bool FOCAL>
 __global__ void __launch_bounds__(1024) head_fwd_long_kernel(const float* __restrict__ x,
                                                               const float* __restrict__ labels, int64_t rows,
                                                               int64_t cols, float* __restrict__ stats) {
+    constexpr int U = 4;
     __shared__ float lds_m[16], lds_s[16];
     for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
         const float* xr = x + r * cols;
         float mt = -INFINITY, st = 0.f;
-        for (int64_t c = threadIdx.x; c < cols; c += 1024) {
-            const float v = ld_stream1(xr + c);
-            if (v > mt) {
-                st = st * exp_rr(mt - v) + (1.0f + (v - v));
-                mt = v;
-            } else if (v != -INFINITY) {
-                st += exp_rr(v - mt);
+        for (int64_t c0 = (int64_t)threadIdx.x * 4; c0 < cols; c0 += 1024 * 4 * U) {
+            float v[U][4];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                // No branch around the load: past the row's end it takes the
+                // last four floats, and keeps those that are this thread's.
+                const int64_t c = c0 + u * 4096, at = c < cols - 4 ? c : cols - 4;
+                const float4 q = ld_unaligned(xr + at);
+                v[u][0] = q.x; v[u][1] = q.y; v[u][2] = q.z; v[u][3] = q.w;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[u][e] = c < cols && at + e >= c ? v[u][e] : -INFINITY;
             }
+            float m = mt;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m = fmaxf(m, v[u][e]);
+            const float base = m == -INFINITY ? 0.f : m;
+            st *= exp_rr(mt - base);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st += exp_rr(v[u][e] - base);
+            mt = m;
         }
         const float m = block_max_1<1024>(mt, lds_m);
         const float ct = mt == -INFINITY ? 0.f : exp_rr(mt - m);
@@ -246,22 +265,54 @@ __global__ void __launch_bounds__(256) head_bwd_tile_kernel(const float* __restr
     }
 }
 
-// Scalar path (cols % 4 != 0 or unaligned): one workgroup per row.
+// Rows of any length: the same tiles, shifted per row so that the gradient's
+// stores start on a 128-byte line (16 bytes for short rows; the loads then do
+// too, or are 128 bits at 4-byte alignment); the float4s that cross either end
+// of a row go element by element.  Rows of fewer than 256 float4s share a
+// workgroup, 2^lpr_log2 lanes each.  [2048, 50257] cross entropy: 248 -> 147
+// us against a workgroup per row with one float per thread (172 with unshifted
+// tiles, 152 shifted to 16 bytes only); 16384 rows of 13 classes 8.6 -> 4.2 us.
 template <int MODE>
-__global__ void __launch_bounds__(256) head_bwd_kernel(const float* __restrict__ x, const float* __restrict__ labels,
-                                                        const float* __restrict__ stats,
-                                                        const float* __restrict__ loss_grad, float* __restrict__ gx,
-                                                        int acc, int64_t rows, int64_t cols, float alpha) {
+__global__ void __launch_bounds__(256) head_bwd_ragged_kernel(const float* __restrict__ x,
+                                                               const float* __restrict__ labels,
+                                                               const float* __restrict__ stats,
+                                                               const float* __restrict__ loss_grad,
+                                                               float* __restrict__ gx, int acc, int64_t rows,
+                                                               int64_t cols, float alpha, int lpr_log2,
+                                                               unsigned lead_mask) {
     const float scale = loss_grad[0] / (float)rows;
-    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+    const int lane = (int)threadIdx.x & ((1 << lpr_log2) - 1), sub = (int)threadIdx.x >> lpr_log2;
+    const int64_t rpb = 256 >> lpr_log2;
+    // The grid is (tiles, row groups): no division.
+    for (int64_t r0 = (int64_t)blockIdx.y * rpb; r0 < rows; r0 += (int64_t)gridDim.y * rpb) {
+        const int64_t r = r0 + sub;
+        if (r >= rows) continue;
+        const int lead = (int)((((uintptr_t)gx >> 2) + (uintptr_t)(r * cols)) & lead_mask);
+        const int64_t c0 = ((int64_t)blockIdx.x * 256 + lane) * 4 - lead;
+        if (c0 >= cols) continue;
         const HeadRow h = head_row<MODE>(stats, labels[r], r, cols, scale);
         const float* xr = x + r * cols;
         float* gr = gx + r * cols;
-        for (int64_t c = threadIdx.x; c < cols; c += 256) {
-            const float xv = MODE != kOneHot ? ld_stream1(xr + c) : 0.f;
-            float d = head_elem<MODE>(xv, c == h.lab, h, scale, alpha);
-            if (acc) d = ld_stream1(gr + c) + d;
-            st_stream1(gr + c, d);
+        if (c0 >= 0 && c0 + 3 < cols) {
+            const float4 xv = MODE != kOneHot ? ld_unaligned(xr + c0) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 ov = acc ? ld_stream(gr + c0) : make_float4(0.f, 0.f, 0.f, 0.f);
+            float d0 = head_elem<MODE>(xv.x, c0 == h.lab, h, scale, alpha);
+            float d1 = head_elem<MODE>(xv.y, c0 + 1 == h.lab, h, scale, alpha);
+            float d2 = head_elem<MODE>(xv.z, c0 + 2 == h.lab, h, scale, alpha);
+            float d3 = head_elem<MODE>(xv.w, c0 + 3 == h.lab, h, scale, alpha);
+            if (acc) {
+                d0 = ov.x + d0; d1 = ov.y + d1; d2 = ov.z + d2; d3 = ov.w + d3;
+            }
+            st_stream(gr + c0, make_float4(d0, d1, d2, d3));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int64_t c = c0 + e;
+                if (c < 0 || c >= cols) continue;
+                float d = head_elem<MODE>(MODE != kOneHot ? ld_stream1(xr + c) : 0.f, c == h.lab, h, scale, alpha);
+                if (acc) d = ld_stream1(gr + c) + d;
+                st_stream1(gr + c, d);
+            }
         }
     }
 }
@@ -513,14 +564,24 @@ template <int MODE>
 int launch_head_bwd(const float* x, const float* labels, const float* stats, const float* loss_grad, float* gx,
                     int acc, int64_t rows, int64_t cols, float alpha, const char* what) {
     const bool vec = cols % 4 == 0 && aligned16(gx) && (MODE == kOneHot || aligned16(x));
-    dim3 grid((unsigned)std::min<int64_t>(rows, (int64_t)num_cus() * 8));
     const int64_t tiles = (cols / 4 + 255) / 256;
-    if (vec && rows * tiles < ((int64_t)1 << 32)) {
+    // Aligned rows of at least 128 float4s keep a tile of their own: 22.4 us
+    // against 29.8 at [16384, 1000].
+    if (vec && cols >= 4 * 128 && rows * tiles < ((int64_t)1 << 32)) {
         launch_kernel((head_bwd_tile_kernel<MODE>), dim3(grid_for(rows * tiles, 1, 1 << 12)), dim3(256), 0,
                       stream(), x, labels, stats, loss_grad, gx, acc, rows, cols, alpha);
-    } else
-        launch_kernel((head_bwd_kernel<MODE>), grid, dim3(256), 0, stream(), x, labels, stats, loss_grad, gx,
-                      acc, rows, cols, alpha);
+    } else {
+        // Long rows shift to whole 128-byte lines, short ones to 16 bytes; n4:
+        // float4s of a row at any shift.
+        const unsigned mask = cols >= 1024 ? 31u : 3u;
+        const int64_t n4 = (cols + mask + 3) / 4;
+        int lg = 0;
+        while (lg < 8 && (1 << lg) < n4) ++lg;
+        const int64_t groups = (rows + (256 >> lg) - 1) / (256 >> lg);
+        const dim3 grid((unsigned)((n4 + 255) / 256), (unsigned)std::min<int64_t>(groups, 65535));
+        launch_kernel((head_bwd_ragged_kernel<MODE>), grid, dim3(256), 0, stream(), x, labels, stats, loss_grad, gx,
+                      acc, rows, cols, alpha, lg, mask);
+    }
     return check_launch(what);
 }
 
