@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_helpers import _offset_dev, binary_bwd, binary_fwd, gemm, rng_normal, rng_uniform
+from gpu_helpers import (_offset_dev, batchnorm_bwd, batchnorm_fwd, binary_bwd, binary_fwd, gemm, rng_normal,
+                         rng_uniform)
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-5
@@ -129,3 +130,32 @@ def test_cross_entropy_rows_at_any_alignment(wm, rows, cols, offset):
         assert ok, f"{w:.3g}x tolerance (accumulate {acc})"
         assert np.array_equal(got[:offset], buf[:offset])
         assert np.array_equal(got[offset + rows * cols:], buf[offset + rows * cols:])
+
+
+# Channels at the ends of each register tile (256 or 1024 threads, 1 to 4
+# float4s or 8 floats each) and just past the largest, planes of one float,
+# of less than a wave and across workgroup steps.
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("shape", [(1, 2, 1, 1), (255, 2, 1, 1), (257, 3, 1, 1), (64, 5, 2, 2), (4, 3, 32, 32),
+                                   (4, 3, 36, 32), (16, 2, 32, 32), (17, 2, 32, 32), (91, 3, 9, 10), (92, 3, 9, 10),
+                                   (200, 2, 7, 7), (40, 70, 14, 14), (3, 2, 200, 100)])
+def test_batchnorm_channel_sizes(wm, shape, accumulate):
+    s = seed_of("bn", shape)
+    o64, oab, ch = oracle.get("f64"), oracle.get("abs"), shape[1]
+    x, g = rng_normal(shape, s) + np.float32(0.5), rng_normal(shape, s + 1)
+    gamma, beta = rng_uniform((ch,), s + 2, 0.5, 1.5), rng_normal((ch,), s + 3)
+    rm, rv = rng_normal((ch,), s + 4), rng_uniform((ch,), s + 5, 0.5, 1.5)
+    y, mean, inv, rm1, rv1 = batchnorm_fwd(x, gamma, beta, rm, rv, True)
+    y64, m64, i64, rm64, rv64 = o64.batchnorm2d(x, gamma, beta, rm, rv, training=True)
+    xs = np.abs(x).mean((0, 2, 3))
+    for got, ref, scale in ((y, y64, oab.batchnorm2d(x, gamma, beta, rm, rv, training=True)[0]), (mean, m64, xs),
+                            (inv, i64, i64), (rm1, rm64, 0.9 * np.abs(rm) + 0.1 * xs), (rv1, rv64, rv64)):
+        ok, w = oracle.close_scaled(got, ref, scale, RTOL, 1e-30)
+        assert ok, f"forward {w:.3g}x tolerance"
+    g0 = (rng_normal(shape, s + 6), rng_normal((ch,), s + 7), rng_normal((ch,), s + 8)) if accumulate else (None,) * 3
+    got = batchnorm_bwd(g, x, gamma, mean, inv, *g0)
+    ref, scale = o64.batchnorm2d_bwd(g, x, gamma, mean, inv), oab.batchnorm2d_bwd(g, x, gamma, mean, inv)
+    for k in range(3):
+        z = g0[k] if accumulate else np.float32(0)
+        ok, w = oracle.close_scaled(got[k], ref[k] + z, scale[k] + np.abs(z), RTOL, 1e-30)
+        assert ok, f"gradient {k} {w:.3g}x tolerance"
