@@ -7,8 +7,8 @@ import numpy as np
 import pytest
 
 import oracle
-from gpu_helpers import (_offset_dev, batchnorm_bwd, batchnorm_fwd, binary_bwd, binary_fwd, gemm, rng_normal,
-                         rng_uniform)
+from gpu_helpers import (_offset_dev, batchnorm_bwd, batchnorm_fwd, binary_bwd, binary_fwd, gemm,
+                         layernorm_bwd, layernorm_fwd, rng_normal, rng_uniform)
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-5
@@ -155,6 +155,28 @@ def test_batchnorm_channel_sizes(wm, shape, accumulate):
     g0 = (rng_normal(shape, s + 6), rng_normal((ch,), s + 7), rng_normal((ch,), s + 8)) if accumulate else (None,) * 3
     got = batchnorm_bwd(g, x, gamma, mean, inv, *g0)
     ref, scale = o64.batchnorm2d_bwd(g, x, gamma, mean, inv), oab.batchnorm2d_bwd(g, x, gamma, mean, inv)
+    for k in range(3):
+        z = g0[k] if accumulate else np.float32(0)
+        ok, w = oracle.close_scaled(got[k], ref[k] + z, scale[k] + np.abs(z), RTOL, 1e-30)
+        assert ok, f"gradient {k} {w:.3g}x tolerance"
+
+
+# Rows at the ends of each LayerNorm tile (1 to 4 float4s of a wave, 256 and
+# 1024 threads), odd lengths, and few or many rows per workgroup.
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("rows,n", [(1, 1), (3, 7), (35, 74), (9, 256), (5, 257), (1100, 512), (33, 768), (300, 767),
+                                    (2100, 1024), (7, 1025), (12, 2048), (5, 2052), (9, 4100), (10, 8192)])
+def test_layernorm_row_lengths(wm, rows, n, accumulate):
+    s = seed_of("ln", rows, n)
+    o64, oab = oracle.get("f64"), oracle.get("abs")
+    x, g = rng_normal((rows, n), s), rng_normal((rows, n), s + 1)
+    gamma, beta = rng_uniform((n,), s + 2, 0.5, 1.5), rng_normal((n,), s + 3)
+    y, mean, inv = layernorm_fwd(x, gamma, beta)
+    ok, w = oracle.close_scaled(y, o64.layernorm(x, gamma, beta)[0], oab.layernorm(x, gamma, beta)[0], RTOL, 1e-30)
+    assert ok, f"forward {w:.3g}x tolerance"
+    g0 = (rng_normal((rows, n), s + 4), rng_normal((n,), s + 5), rng_normal((n,), s + 6)) if accumulate else (None,) * 3
+    got = layernorm_bwd(g, x, gamma, mean, inv, *g0)
+    ref, scale = o64.layernorm_bwd(g, x, gamma, mean, inv), oab.layernorm_bwd(g, x, gamma, mean, inv)
     for k in range(3):
         z = g0[k] if accumulate else np.float32(0)
         ok, w = oracle.close_scaled(got[k], ref[k] + z, scale[k] + np.abs(z), RTOL, 1e-30)

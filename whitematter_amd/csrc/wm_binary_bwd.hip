@@ -186,7 +186,7 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
 // out[o, c] (+)= sum_k part[o, k, c], k in 0..K-1.  A workgroup owns S adjacent
 // columns of one o and its threads form G = 256 / S groups: group g folds partial
 // rows k = g, g + G, g + 2G, ... (8 interleaved accumulators, combined in a
-// fixed order), and the G group sums are added in group order through LDS.
+// fixed order), and the G group sums are added in a tree through LDS.
 // S is chosen so the grid has ~256 workgroups or more: with few columns
 // and many partial rows (a Linear bias gradient, 1024 columns over 1024
 // row groups) 64-column workgroups left 16 workgroups each walking 256
@@ -212,13 +212,14 @@ __global__ void __launch_bounds__(kBlock) colsum_finalize_kernel(const float* __
             for (int j = 0; k < K; k += G, ++j) s[j & 7] += pt[k * C + c];
         }
         lds[g][cl] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
-        __syncthreads();
-        if (g == 0 && c < C) {
-            float t = lds[0][cl];
 #pragma unroll
-            for (int gg = 1; gg < G; ++gg) t += lds[gg][cl];
+        for (int h = G / 2; h > 0; h /= 2) {
+            __syncthreads();
+            if (g < h) lds[g][cl] += lds[g + h][cl];
+        }
+        if (g == 0 && c < C) {
             float* dst = out + ou * C + c;
-            *dst = acc ? *dst + t : t;
+            *dst = acc ? *dst + lds[0][cl] : lds[0][cl];
         }
         __syncthreads();
     }

@@ -199,68 +199,123 @@ __global__ void __launch_bounds__(NT, (ln_bwd_min_waves<NT, ITEMS>())) ln_bwd_ke
         }
 }
 
-// Column sums of [parts, n] partials: out[c] (+)= sum_w part[w][c], w in
-// order.  64 columns per workgroup; the 4 waves take every 4th partial row
-// and combine in LDS.  blockIdx.z picks one of two independent sums (the
-// weight and bias gradients share the launch).
+// Rows of up to 1024 elements: a wave per row (no barrier inside a row), four
+// rows of a workgroup at a time.  The four waves' parameter partials are added
+// through LDS at the end, so a workgroup leaves one partial row for four
+// waves' worth of rows in flight.  [8192, 768]: 17 us against 36.6
+// for a 256-thread workgroup per row (32 rows each; 17.9 with 8 rows each, and
+// 10 more for the sums over its four times as many partial rows).
+template <int ITEMS, bool VEC>
+__global__ void __launch_bounds__(256) ln_bwd_wave_kernel(const float* __restrict__ g, const float* __restrict__ x,
+                                                           const float* __restrict__ gamma,
+                                                           const float* __restrict__ mean,
+                                                           const float* __restrict__ inv_std, int64_t rows, int64_t n,
+                                                           float* __restrict__ gx, int acc, float* __restrict__ pgamma,
+                                                           float* __restrict__ pbeta) {
+    using Tile = RowTile<64, ITEMS, VEC>;
+    __shared__ float lds[4][ITEMS * 256];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    Tile gt;
+    gt.template load<true>(gamma, n, 0.f);
+    float pg[ITEMS][4], pb[ITEMS][4];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) pg[i][e] = pb[i][e] = 0.f;
+    const float nf = (float)n;
+    for (int64_t r = (int64_t)blockIdx.x * 4 + wave; r < rows; r += (int64_t)gridDim.x * 4) {
+        Tile dy, xv;
+        dy.load(g + r * n, n, 0.f);
+        xv.load(x + r * n, n, 0.f);
+        const float m = mean[r], iv = inv_std[r];
+        float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float xn = (xv.v[i][e] - m) * iv;
+                xv.v[i][e] = xn;
+                const float dg = dy.v[i][e] * gt.v[i][e];
+                s1 += dg;
+                s2 += dg * xn;
+                pg[i][e] += dy.v[i][e] * xn;  // padding: dy = 0
+                pb[i][e] += dy.v[i][e];
+            }
+        if (gx) {
+            const float mdg = wave_sum(s1) / nf, mdgx = wave_sum(s2) / nf;
+#pragma unroll
+            for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    dy.v[i][e] = iv * (dy.v[i][e] * gt.v[i][e] - mdg - xv.v[i][e] * mdgx);
+            if (acc) {
+                Tile old;
+                old.load(gx + r * n, n, 0.f);
+#pragma unroll
+                for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dy.v[i][e] = old.v[i][e] + dy.v[i][e];
+            }
+            dy.store(gx + r * n, n);
+        }
+    }
+    auto fold = [&](const float (&p)[ITEMS][4], float* part) {
+        if (!part) return;  // uniform
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) lds[wave][Tile::col(i, e)] = p[i][e];
+        __syncthreads();
+        for (int c = (int)threadIdx.x; c < n; c += 256)
+            part[(int64_t)blockIdx.x * n + c] = (lds[0][c] + lds[1][c]) + (lds[2][c] + lds[3][c]);
+    };
+    fold(pg, pgamma);
+    fold(pb, pbeta);
+}
+
+// Column sums of [parts, n] partials: out[c] (+)= sum_p part[p][c].  A
+// workgroup owns S adjacent columns; its 256 / S row lanes take every
+// (256 / S)-th partial row in 8 interleaved accumulators and are added in a
+// tree through LDS.  blockIdx.z picks one of two independent sums (the weight and
+// bias gradients share the launch).
+template <int S>
 __global__ void __launch_bounds__(256) colsum_parts_kernel(const float* __restrict__ part0,
                                                             const float* __restrict__ part1, int64_t parts, int64_t n,
                                                             float* __restrict__ out0, float* __restrict__ out1,
                                                             int acc0, int acc1) {
-    __shared__ float lds[4][64];
+    constexpr int G = 256 / S;
+    __shared__ float lds[G][S];
     const float* part = blockIdx.z ? part1 : part0;
     float* out = blockIdx.z ? out1 : out0;
     const int acc = blockIdx.z ? acc1 : acc0;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t c = (int64_t)blockIdx.x * 64 + lane;
-    float s = 0.f;
-    if (c < n)
-        for (int64_t p = w; p < parts; p += 4) s += part[p * n + c];
-    lds[w][lane] = s;
-    __syncthreads();
-    if (w == 0 && c < n) {
-        const float t = (lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane]);
-        out[c] = acc ? out[c] + t : t;
-    }
-}
-
-// First stage for many partial rows: workgroup (x, y, z) sums partial rows
-// [y * chunk, (y + 1) * chunk) of 64 columns of sum z into out2_z[y][c]; each
-// wave takes every 4th row with four independent accumulators (loads in
-// flight), the waves combine in LDS in a fixed order.  colsum_parts_kernel
-// then sums the out2 rows.
-__global__ void __launch_bounds__(256) colsum_stage_kernel(const float* __restrict__ part0,
-                                                            const float* __restrict__ part1, int64_t parts, int64_t n,
-                                                            int64_t chunk, float* __restrict__ out2_0,
-                                                            float* __restrict__ out2_1) {
-    __shared__ float lds[4][64];
-    const float* part = blockIdx.z ? part1 : part0;
-    float* out2 = blockIdx.z ? out2_1 : out2_0;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t c = (int64_t)blockIdx.x * 64 + lane;
-    const int64_t p0 = (int64_t)blockIdx.y * chunk;
-    const int64_t p1 = p0 + chunk < parts ? p0 + chunk : parts;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+    const int cl = threadIdx.x % S, g = threadIdx.x / S;
+    const int64_t c = (int64_t)blockIdx.x * S + cl;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (c < n) {
-        int64_t p = p0 + w;
-        for (; p + 12 < p1; p += 16) {
-            a0 += part[p * n + c];
-            a1 += part[(p + 4) * n + c];
-            a2 += part[(p + 8) * n + c];
-            a3 += part[(p + 12) * n + c];
+        int64_t p = g;
+        for (; p + 7 * G < parts; p += 8 * G) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[j] += part[(p + j * G) * n + c];
         }
-        for (; p < p1; p += 4) a0 += part[p * n + c];
+#pragma unroll
+        for (int j = 0; j < 7; ++j, p += G)
+            if (p < parts) s[j] += part[p * n + c];
     }
-    lds[w][lane] = (a0 + a1) + (a2 + a3);
-    __syncthreads();
-    if (w == 0 && c < n) out2[(int64_t)blockIdx.y * n + c] = (lds[0][lane] + lds[1][lane]) + (lds[2][lane] + lds[3][lane]);
+    lds[g][cl] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+#pragma unroll
+    for (int h = G / 2; h > 0; h /= 2) {
+        __syncthreads();
+        if (g < h) lds[g][cl] += lds[g + h][cl];
+    }
+    if (g == 0 && c < n) out[c] = acc ? out[c] + lds[0][cl] : lds[0][cl];
 }
 
 // Column sums of [parts, n] partial rows into out_g and out_b (+= when
-// acc_*; a null partial array skips its sum): one pass for up to 64 rows,
-// else colsum_stage_kernel first.  Both sums share each launch, so the
-// weight and bias gradients cost two dispatches, not four (LayerNorm
-// backward at [32768, 4096]: 283.5-284.1 -> 278.0-280.8 us).
+// acc_*; a null partial array skips its sum), in one launch.  As many columns
+// per workgroup as leave one workgroup per CU, so that few columns over many
+// partial rows still spread over the chip (a stage of 64-row sums in front
+// cost a second dispatch: 8.5 -> 4.5 us at [256, 768] partials).
 int colsum_parts(const float* part_g, float* out_g, int acc_g, const float* part_b, float* out_b, int acc_b,
                  int64_t parts, int64_t n, const char* what) {
     hipStream_t st = stream();
@@ -270,22 +325,14 @@ int colsum_parts(const float* part_g, float* out_g, int acc_g, const float* part
     }
     if (!part_g) return WM_OK;
     const unsigned jobs = part_b ? 2u : 1u;
-    const dim3 cg((unsigned)((n + 63) / 64), 1u, jobs);
-    if (parts <= 64) {
-        launch_kernel(colsum_parts_kernel, cg, dim3(256), 0, st, part_g, part_b, parts, n, out_g, out_b, acc_g,
-                      acc_b);
-        return check_launch(what);
-    }
-    const int64_t chunk = 64, parts2 = (parts + chunk - 1) / chunk;
-    Workspace w2((size_t)(jobs * parts2 * n) * sizeof(float));
-    if (!w2.p) return set_error(WM_ERR_NOMEM, std::string(what) + ": workspace");
-    float* s0 = w2.as<float>();
-    float* s1 = jobs == 2 ? s0 + parts2 * n : nullptr;
-    launch_kernel(colsum_stage_kernel, dim3(cg.x, (unsigned)parts2, jobs), dim3(256), 0, st, part_g, part_b, parts,
-                  n, chunk, s0, s1);
-    WM_TRY(check_launch(what));
-    launch_kernel(colsum_parts_kernel, cg, dim3(256), 0, st, (const float*)s0, (const float*)s1, parts2, n, out_g,
-                  out_b, acc_g, acc_b);
+    const int64_t cols = n * jobs, want = num_cus();
+#define WM_CP(S)                                                                                              \
+    launch_kernel(colsum_parts_kernel<S>, dim3((unsigned)((n + S - 1) / S), 1u, jobs), dim3(256), 0, st, part_g, \
+                  part_b, parts, n, out_g, out_b, acc_g, acc_b)
+    if (cols >= 64 * want) WM_CP(64);
+    else if (cols >= 16 * want) WM_CP(16);
+    else WM_CP(4);
+#undef WM_CP
     return check_launch(what);
 }
 
@@ -1012,13 +1059,14 @@ __global__ void __launch_bounds__(256) dropout_mask_kernel(float* __restrict__ m
 // host
 // ---------------------------------------------------------------------------
 
-// LayerNorm register tiles: NT in {64, 256, 1024}, ITEMS in {1, 2}; rows
-// over 8192 elements take the streaming path (nt == 0).
+// LayerNorm register tiles: a wave with up to 4 float4s per lane (1024
+// columns), else 256 or 1024 threads with up to 2; rows over 8192 elements
+// take the streaming path (nt == 0).
 TileChoice ln_tile(int64_t n) {
     TileChoice t;
     const int nts[3] = {64, 256, 1024};
     for (int nt : nts)
-        for (int items = 1; items <= 2; ++items)
+        for (int items = 1; items <= (nt == 64 ? 4 : 2); ++items)
             if (n <= (int64_t)nt * 4 * items) {
                 t.nt = nt;
                 t.items = items;
@@ -1050,7 +1098,7 @@ int launch_ln_fwd(const float* x, const float* gamma, const float* beta, int64_t
                                n, eps, y, mean, inv);                                                           \
         return check_launch("wm_layernorm_fwd");                                                                \
     }
-    WM_LNF(64, 1) WM_LNF(64, 2) WM_LNF(256, 1) WM_LNF(256, 2) WM_LNF(1024, 1) WM_LNF(1024, 2)
+    WM_LNF(64, 1) WM_LNF(64, 2) WM_LNF(64, 3) WM_LNF(64, 4) WM_LNF(256, 2) WM_LNF(1024, 1) WM_LNF(1024, 2)
 #undef WM_LNF
     return set_error(WM_ERR_INVALID, "wm_layernorm_fwd: no tile");
 }
@@ -1080,9 +1128,18 @@ int launch_ln_bwd(const float* g, const float* x, const float* gamma, const floa
                             dbeta, acc_b, chunks, n, "wm_layernorm_bwd(colsum)");
     }
     // Fused path: G workgroups, each leaving one [n] partial per parameter
-    // gradient.  G also bounds the partial traffic: at least 32 rows each.
-    int64_t G = std::min<int64_t>(rows, (int64_t)num_cus() * ln_waves(tc.nt) * 2);
-    if (want_p) G = std::max<int64_t>(1, std::min<int64_t>(G, (rows + 31) / 32));
+    // gradient.  With parameter gradients a wave-per-row workgroup takes at
+    // least 8 rows (two per wave) and the grid stops at one workgroup per CU
+    // (four for rows of one float4 per lane, which keep fewer bytes in
+    // flight): [8192, 768] 17.3 + 4.5 us for the two dispatches, against 16.7 + 6.2
+    // at two per CU and 17.2 + 9.8 at four; [32768, 128] 12.9 + 4.4 at four
+    // against 27.9 + 4.5 at one.  Wider rows: at least 8 rows per workgroup, or 4
+    // when there are few (of 32 before: [768, 8192] 82 -> 23 us).
+    const bool wave = tc.nt == 64;
+    const int per_cu = !wave ? ln_waves(tc.nt) * 2 : want_p && tc.items > 1 ? 1 : 4;
+    int64_t G = std::min<int64_t>(wave ? (rows + 3) / 4 : rows, (int64_t)num_cus() * per_cu);
+    const int64_t least = wave || rows >= 1024 ? 8 : 4;
+    if (want_p) G = std::max<int64_t>(1, std::min<int64_t>(G, (rows + least - 1) / least));
     Workspace wg(dgamma ? (size_t)(G * n) * sizeof(float) : 0);
     Workspace wb(dbeta ? (size_t)(G * n) * sizeof(float) : 0);
     if ((dgamma && !wg.p) || (dbeta && !wb.p)) return set_error(WM_ERR_NOMEM, "wm_layernorm_bwd: workspace");
@@ -1099,8 +1156,20 @@ int launch_ln_bwd(const float* g, const float* x, const float* gamma, const floa
                                rows, n, gx, acc_x, wg.as<float>(), wb.as<float>());                             \
         launched = true;                                                                                        \
     }
-    WM_LNB(64, 1) WM_LNB(64, 2) WM_LNB(256, 1) WM_LNB(256, 2) WM_LNB(1024, 1) WM_LNB(1024, 2)
+    WM_LNB(256, 2) WM_LNB(1024, 1) WM_LNB(1024, 2)
 #undef WM_LNB
+#define WM_LNW(IT)                                                                                                  \
+    if (!launched && wave && tc.items == IT) {                                                                      \
+        if (vec)                                                                                                    \
+            launch_kernel((ln_bwd_wave_kernel<IT, true>), grid, dim3(256), 0, st, g, x, gamma, mean, inv, rows, n,  \
+                          gx, acc_x, wg.as<float>(), wb.as<float>());                                               \
+        else                                                                                                        \
+            launch_kernel((ln_bwd_wave_kernel<IT, false>), grid, dim3(256), 0, st, g, x, gamma, mean, inv, rows, n, \
+                          gx, acc_x, wg.as<float>(), wb.as<float>());                                               \
+        launched = true;                                                                                            \
+    }
+    WM_LNW(1) WM_LNW(2) WM_LNW(3) WM_LNW(4)
+#undef WM_LNW
     if (!launched) return set_error(WM_ERR_INVALID, "wm_layernorm_bwd: no tile");
     WM_TRY(check_launch("wm_layernorm_bwd"));
     return colsum_parts(dgamma ? wg.as<float>() : nullptr, dgamma, acc_g, dbeta ? wb.as<float>() : nullptr, dbeta,

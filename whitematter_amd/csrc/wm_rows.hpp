@@ -28,8 +28,10 @@ template <int NT, int ITEMS, bool VEC>
 struct RowTile {
     float v[ITEMS][4];
 
+    // The row's NT threads: the workgroup, or (NT = 64) one of its waves.
     __device__ __forceinline__ static int64_t col(int t, int e) {
-        return VEC ? ((int64_t)(t * NT + (int)threadIdx.x) * 4 + e) : ((int64_t)t * NT * 4 + (int64_t)e * NT + threadIdx.x);
+        const int i = (int)threadIdx.x & (NT - 1);
+        return VEC ? ((int64_t)(t * NT + i) * 4 + e) : ((int64_t)t * NT * 4 + (int64_t)e * NT + i);
     }
 
     // CACHED = false: non-temporal loads (data read once); true: ordinary
