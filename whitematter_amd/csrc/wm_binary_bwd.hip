@@ -184,34 +184,24 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
 }
 
 // out[o, c] (+)= sum_k part[o, k, c], k in 0..K-1.  A workgroup owns S adjacent
-// columns of one o and its threads form G = 256 / S groups: group g folds partial
-// rows k = g, g + G, g + 2G, ... (8 interleaved accumulators, combined in a
-// fixed order), and the G group sums are added in a tree through LDS.
-// S is chosen so the grid has ~256 workgroups or more: with few columns
-// and many partial rows (a Linear bias gradient, 1024 columns over 1024
-// row groups) 64-column workgroups left 16 workgroups each walking 256
-// rows per wave (13.6 us).
-template <int S>
-__global__ void __launch_bounds__(kBlock) colsum_finalize_kernel(const float* __restrict__ part, float* __restrict__ out,
+// columns of one o and its NT threads form G = NT / S groups: group g folds
+// partial rows k = g, g + G, g + 2G, ... (8 interleaved accumulators, combined
+// in a fixed order), and the G group sums are added in a tree through LDS.
+// Few columns over many partial rows (a Linear bias gradient, 1024 columns
+// over 1024 row groups) take 4 columns per workgroup, so that the grid has
+// ~256 workgroups (64 columns left 16 workgroups each walking 256 rows per
+// wave: 13.6 us); from 2048 columns on, 64 columns with 16 groups read whole
+// lines with as many rows in flight ([512, 4096] partials 5.2 us against 11.5
+// for 16 columns with 16 groups).
+template <int S, int NT>
+__global__ void __launch_bounds__(NT) colsum_finalize_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                                   int acc, int64_t K, int64_t C, int64_t O) {
-    constexpr int G = kBlock / S;
+    constexpr int G = NT / S;
     __shared__ float lds[G][S];
     const int cl = threadIdx.x % S, g = threadIdx.x / S;
-    const int64_t tiles = (C + S - 1) / S;
-    for (int64_t item = blockIdx.x; item < O * tiles; item += gridDim.x) {
-        const int64_t ou = item / tiles;
-        const int64_t c = (item - ou * tiles) * S + cl;
-        const float* pt = part + ou * K * C;
-        float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (c < C) {
-            int64_t k = g;
-            for (; k + 7 * G < K; k += 8 * G) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) s[j] += pt[(k + j * G) * C + c];
-            }
-            for (int j = 0; k < K; k += G, ++j) s[j & 7] += pt[k * C + c];
-        }
-        lds[g][cl] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    for (int64_t ou = blockIdx.y; ou < O; ou += gridDim.y) {
+        const int64_t c = (int64_t)blockIdx.x * S + cl;
+        lds[g][cl] = c < C ? strided_sum<G>(part + ou * K * C + c, C, g, K) : 0.f;
 #pragma unroll
         for (int h = G / 2; h > 0; h /= 2) {
             __syncthreads();
@@ -228,12 +218,13 @@ __global__ void __launch_bounds__(kBlock) colsum_finalize_kernel(const float* __
 // colsum_finalize_kernel with its column slot width chosen for C.
 int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, int64_t C, int64_t O, hipStream_t st) {
     const int64_t want = (int64_t)num_cus(), cols = C * O;
-#define WM_CF(S)                                                                                             \
-    launch_kernel(colsum_finalize_kernel<S>, dim3(grid_for((C + S - 1) / S * O, 1, 8)), dim3(kBlock), 0, st, \
-                  part, out, acc, K, C, O)
-    if (cols >= 64 * want) WM_CF(64);
-    else if (cols >= 16 * want) WM_CF(16);
-    else WM_CF(4);
+#define WM_CF(S, NT)                                                                                      \
+    launch_kernel((colsum_finalize_kernel<S, NT>),                                                        \
+                  dim3((unsigned)((C + S - 1) / S), (unsigned)std::min<int64_t>(O, 65535)), dim3(NT), 0, st, part, \
+                  out, acc, K, C, O)
+    if (cols >= 64 * want) WM_CF(64, kBlock);
+    else if (cols >= 8 * want) WM_CF(64, 1024);
+    else WM_CF(4, kBlock);
 #undef WM_CF
     return check_launch("wm_binary_bwd(colsum finalize)");
 }

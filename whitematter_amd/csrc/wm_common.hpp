@@ -231,6 +231,27 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
+// Sum of column values p[k * ld], k = g, g + G, g + 2G, ... < K, in 8
+// interleaved accumulators combined in a fixed order.  Eight loads go out
+// before the first is added (written as one expression per term, the compiler
+// waited for each); past K the last batch reads term K - 1 and adds 0.
+template <int G>
+__device__ __forceinline__ float strided_sum(const float* p, int64_t ld, int g, int64_t K) {
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int64_t k = g; k < K; k += 8 * G) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t kj = k + j * G;
+            v[j] = p[(kj < K ? kj : K - 1) * ld];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[j] += k + j * G < K ? v[j] : 0.f;
+    }
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 // Block-wide sum for blockDim.x == NT (multiple of 64).  `lds` must hold
 // NT/64 floats.  Every thread gets the total; order is fixed.
 template <int NT>

@@ -200,8 +200,9 @@ __global__ void __launch_bounds__(NT) epilogue_fwd_wg_kernel(uint16_t* __restric
     }
 }
 
-// Backward: a workgroup owns 8*kBlock adjacent columns and row group k
-// (blockIdx.y of K = gridDim.y), the rows k, k + K, k + 2K, ...: the resident
+// Backward: a workgroup owns up to 8*kBlock adjacent columns (512 per wave) and
+// row group k (blockIdx.y of K = gridDim.y), the rows k, k + K, k + 2K, ...
+// (of row blocks, when its waves share out the rows): the resident
 // workgroups then read one narrow band of rows that advances down the
 // matrix (67.6 -> 73.4 % of the HBM peak at config 5 against contiguous
 // blocks of rows / K rows).  With 128-bit accesses lane i of wave w handles
@@ -220,41 +221,50 @@ __device__ __forceinline__ void load_half4(const uint16_t* p, float* out) {
     out[3] = half_bits_to_float(q.y >> 16);
 }
 
-template <bool VEC, bool FC>
+// FULL: cols is a multiple of 512, every lane's columns exist.
+template <bool VEC, bool FC, bool FULL>
 __global__ void __launch_bounds__(kBlock) epilogue_bwd_kernel(const float* __restrict__ dm,
                                                                const uint16_t* __restrict__ h,
                                                                const uint16_t* __restrict__ res,
                                                                const float* __restrict__ g, float* __restrict__ gh,
                                                                int acc_h, float* __restrict__ gres, int acc_res,
                                                                float* __restrict__ part, int64_t rows, int64_t cols,
-                                                               float lo, float hi) {
+                                                               float lo, float hi, int wpr_log2) {
     constexpr int W = VEC ? 8 : 1;
+    __shared__ float lds[kBlock][W];
+    // 2^wpr_log2 waves side by side along a row, the workgroup's other waves on
+    // the next rows.
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int wpr = 1 << wpr_log2, rpb = (kBlock / 64) >> wpr_log2, sub = w >> wpr_log2;
     int64_t cg[2];  // first column of each 4-column group (VEC), or the one column
+    const int64_t tile = (int64_t)blockIdx.x * wpr + (w & (wpr - 1));
     if constexpr (VEC) {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-        cg[0] = (int64_t)blockIdx.x * (kBlock * 8) + w * 512 + lane * 4;
+        cg[0] = tile * 512 + lane * 4;
         cg[1] = cg[0] + 256;
-        if (cg[0] >= cols) return;  // cols % 512 == 0 on this path: both groups are in range
     } else {
-        cg[0] = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-        if (cg[0] >= cols) return;
+        cg[0] = tile * 64 + lane;
+        cg[1] = cg[0];
     }
+    const bool in0 = FULL || cg[0] < cols, in1 = FULL || (VEC && cg[1] < cols);
     float gv[W], acc[W];
 #pragma unroll
     for (int j = 0; j < W; ++j) {
-        gv[j] = VEC ? g[cg[j / 4] + (j % 4)] : g[cg[0]];
+        gv[j] = (VEC && j >= 4 ? in1 : in0) ? g[cg[j / 4] + (j % 4)] : 0.f;
         acc[j] = 0.f;
     }
 #pragma unroll 2
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    for (int64_t r = (int64_t)blockIdx.y * rpb + sub; r < rows; r += (int64_t)gridDim.y * rpb) {
+        if (!in0) break;
         const float dw = dm[r];
         const int64_t roff = r * cols;
         float hv[W], rv[W];
         if constexpr (VEC) {
+            // The second group past the row's end repeats the first (not used).
+            const int64_t c1 = in1 ? cg[1] : cg[0];
             load_half4(h + roff + cg[0], hv);
-            load_half4(h + roff + cg[1], hv + 4);
+            load_half4(h + roff + c1, hv + 4);
             load_half4(res + roff + cg[0], rv);
-            load_half4(res + roff + cg[1], rv + 4);
+            load_half4(res + roff + c1, rv + 4);
         } else {
             hv[0] = half_bits_to_float(h[roff + cg[0]]);
             rv[0] = half_bits_to_float(res[roff + cg[0]]);
@@ -271,6 +281,7 @@ __global__ void __launch_bounds__(kBlock) epilogue_bwd_kernel(const float* __res
         if constexpr (VEC) {
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
+                if (q && !in1) break;
                 const int64_t off = roff + cg[q];
                 const float4 d = make_float4(dt[4 * q], dt[4 * q + 1], dt[4 * q + 2], dt[4 * q + 3]);
                 if (gh) {
@@ -296,49 +307,27 @@ __global__ void __launch_bounds__(kBlock) epilogue_bwd_kernel(const float* __res
             if (gres) gres[off] = acc_res ? gres[off] + dt[0] : dt[0];
         }
     }
-    if (part) {
-        float* pr = part + (int64_t)blockIdx.y * cols;
-        if constexpr (VEC) {
-            *reinterpret_cast<float4*>(pr + cg[0]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-            *reinterpret_cast<float4*>(pr + cg[1]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
-        } else {
-            pr[cg[0]] = acc[0];
-        }
+    if (!part) return;
+    if (rpb > 1) {  // the workgroup's rows, in order
+#pragma unroll
+        for (int j = 0; j < W; ++j) lds[threadIdx.x][j] = acc[j];
+        __syncthreads();
+        if (sub) return;
+        for (int q = 1; q < rpb; ++q)
+#pragma unroll
+            for (int j = 0; j < W; ++j) acc[j] += lds[threadIdx.x + q * wpr * 64][j];
+    }
+    float* pr = part + (int64_t)blockIdx.y * cols;
+    if constexpr (VEC) {
+        if (in0) *reinterpret_cast<float4*>(pr + cg[0]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+        if (in1) *reinterpret_cast<float4*>(pr + cg[1]) = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    } else {
+        if (in0) pr[cg[0]] = acc[0];
     }
 }
 
-// gg[c] (+)= sum_k part[k, c]: 64 columns per workgroup of 16 waves; wave
-// w folds k = w, w + 16, ... (four loads in flight per lane), and the 16
-// wave sums are added in wave order through LDS (a fixed order).
-constexpr int kSumBlock = 1024;
-__global__ void __launch_bounds__(kSumBlock) epilogue_gsum_kernel(const float* __restrict__ part,
-                                                                   float* __restrict__ gg, int acc, int64_t K,
-                                                                   int64_t C) {
-    constexpr int NW = kSumBlock / 64;
-    __shared__ float lds[NW][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int64_t c0 = (int64_t)blockIdx.x * 64; c0 < C; c0 += (int64_t)gridDim.x * 64) {
-        const int64_t c = c0 + lane;
-        float s[4] = {0.f, 0.f, 0.f, 0.f};
-        if (c < C) {
-            int64_t k = w;
-            for (; k + 3 * NW < K; k += 4 * NW) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s[j] += part[(k + j * NW) * C + c];
-            }
-            for (int j = 0; k < K; k += NW, ++j) s[j & 3] += part[k * C + c];
-        }
-        lds[w][lane] = (s[0] + s[1]) + (s[2] + s[3]);
-        __syncthreads();
-        if (w == 0 && c < C) {
-            float t = lds[0][lane];
-#pragma unroll
-            for (int ww = 1; ww < NW; ++ww) t += lds[ww][lane];
-            gg[c] = acc ? gg[c] + t : t;
-        }
-        __syncthreads();
-    }
-}
+// out[c] (+)= sum_k part[k, c], k in 0..K-1 (wm_binary_bwd.hip).
+int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, int64_t C, int64_t O, hipStream_t st);
 
 // The clamp bounds for which the hardware min / max reproduce the
 // reference's compare-and-select clamp (see chain).
@@ -393,31 +382,35 @@ int wm_epilogue_f16_bwd(const float* dm, const uint16_t* h, const uint16_t* res,
     if (!dm || !h || !res || !g) return set_error(WM_ERR_INVALID, "wm_epilogue_f16_bwd: null pointer");
     if (!gh && !gres && !gg) return WM_OK;
     WM_CHECK_INIT();
-    const bool vec = cols % 512 == 0 && aligned16(h) && aligned16(res) && aligned16(g) && (!gh || aligned16(gh)) &&
-                     (!gres || aligned16(gres));
-    const int64_t W = vec ? 8 : 1;
-    const int64_t col_tiles = (cols + kBlock * W - 1) / (kBlock * W);
-    // ~4 workgroups per CU, each row group of at least 16 rows: each thread
-    // folds its columns' dg partials over rows / K rows, and the second pass
-    // reads K partials per column
-    int64_t K = std::min<int64_t>(((int64_t)num_cus() * 4 + col_tiles - 1) / col_tiles, (rows + 15) / 16);
+    const bool vec = cols % 4 == 0 && cols >= 256 && aligned16(h) && aligned16(res) && aligned16(g) &&
+                     (!gh || aligned16(gh)) && (!gres || aligned16(gres));
+    // A wave covers 512 columns (64 of a short or unaligned row); as many waves
+    // side by side along a row as divide it, a workgroup's other waves on the
+    // next rows.
+    const int64_t wave_tiles = (cols + (vec ? 511 : 63)) / (vec ? 512 : 64);
+    const int wpr_log2 = wave_tiles % 4 == 0 ? 2 : wave_tiles % 2 == 0 ? 1 : 0;
+    const int64_t rpb = 4 >> wpr_log2, col_tiles = wave_tiles >> wpr_log2;
+    // ~4 workgroups per CU, each row group of at least 4 rows per wave: each
+    // thread folds its columns' dg partials over its rows, and the second
+    // pass reads K partials per column.  With 16 rows per thread at least and a
+    // whole workgroup per row, [4096, 1024] ran 256 workgroups, half their
+    // lanes idle: 24 -> 14 us; [1024, 4096] 26 -> 14.5 us; [16384, 64], a wave
+    // of whose workgroups had columns, 7.8 -> 5.4 us.
+    int64_t K = std::min<int64_t>(((int64_t)num_cus() * 4 + col_tiles - 1) / col_tiles, (rows + 4 * rpb - 1) / (4 * rpb));
     K = std::max<int64_t>(1, std::min<int64_t>(K, 65535));
     Workspace ws(gg ? (size_t)(K * cols) * sizeof(float) : 0);
     if (gg && !ws.p) return set_error(WM_ERR_NOMEM, "wm_epilogue_f16_bwd: workspace");
     dim3 grid((unsigned)col_tiles, (unsigned)K);
     const bool fc = clamp_is_minmax(lo, hi);
-#define WM_EPI_BWD(V, F)                                                                                     \
-    launch_kernel(epilogue_bwd_kernel<V, F>, grid, dim3(kBlock), 0, stream(), dm, h, res, g, gh, acc_h, gres, \
-                  acc_res, ws.as<float>(), rows, cols, lo, hi)
-    if (vec) { if (fc) WM_EPI_BWD(true, true); else WM_EPI_BWD(true, false); }
-    else { if (fc) WM_EPI_BWD(false, true); else WM_EPI_BWD(false, false); }
+#define WM_EPI_BWD(V, F, A)                                                                                      \
+    launch_kernel((epilogue_bwd_kernel<V, F, A>), grid, dim3(kBlock), 0, stream(), dm, h, res, g, gh, acc_h, gres, \
+                  acc_res, ws.as<float>(), rows, cols, lo, hi, wpr_log2)
+    if (vec && cols % 512 == 0) { if (fc) WM_EPI_BWD(true, true, true); else WM_EPI_BWD(true, false, true); }
+    else if (vec) { if (fc) WM_EPI_BWD(true, true, false); else WM_EPI_BWD(true, false, false); }
+    else { if (fc) WM_EPI_BWD(false, true, false); else WM_EPI_BWD(false, false, false); }
 #undef WM_EPI_BWD
     WM_TRY(check_launch("wm_epilogue_f16_bwd"));
-    if (gg) {
-        launch_kernel(epilogue_gsum_kernel, dim3(grid_for(cols, 64, 8)), dim3(kSumBlock), 0, stream(),
-                      ws.as<float>(), gg, acc_g, K, cols);
-        WM_TRY(check_launch("wm_epilogue_f16_bwd(gsum)"));
-    }
+    if (gg) return launch_colsum_finalize(ws.as<float>(), gg, acc_g, K, cols, 1, stream());
     return WM_OK;
 }
 

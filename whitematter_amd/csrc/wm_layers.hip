@@ -275,34 +275,23 @@ __global__ void __launch_bounds__(256) ln_bwd_wave_kernel(const float* __restric
 }
 
 // Column sums of [parts, n] partials: out[c] (+)= sum_p part[p][c].  A
-// workgroup owns S adjacent columns; its 256 / S row lanes take every
-// (256 / S)-th partial row in 8 interleaved accumulators and are added in a
+// workgroup owns S adjacent columns; its NT / S row lanes take every
+// (NT / S)-th partial row in 8 interleaved accumulators and are added in a
 // tree through LDS.  blockIdx.z picks one of two independent sums (the weight and
 // bias gradients share the launch).
-template <int S>
-__global__ void __launch_bounds__(256) colsum_parts_kernel(const float* __restrict__ part0,
+template <int S, int NT>
+__global__ void __launch_bounds__(NT) colsum_parts_kernel(const float* __restrict__ part0,
                                                             const float* __restrict__ part1, int64_t parts, int64_t n,
                                                             float* __restrict__ out0, float* __restrict__ out1,
                                                             int acc0, int acc1) {
-    constexpr int G = 256 / S;
+    constexpr int G = NT / S;
     __shared__ float lds[G][S];
     const float* part = blockIdx.z ? part1 : part0;
     float* out = blockIdx.z ? out1 : out0;
     const int acc = blockIdx.z ? acc1 : acc0;
     const int cl = threadIdx.x % S, g = threadIdx.x / S;
     const int64_t c = (int64_t)blockIdx.x * S + cl;
-    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (c < n) {
-        int64_t p = g;
-        for (; p + 7 * G < parts; p += 8 * G) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) s[j] += part[(p + j * G) * n + c];
-        }
-#pragma unroll
-        for (int j = 0; j < 7; ++j, p += G)
-            if (p < parts) s[j] += part[p * n + c];
-    }
-    lds[g][cl] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+    lds[g][cl] = c < n ? strided_sum<G>(part + c, n, g, parts) : 0.f;
 #pragma unroll
     for (int h = G / 2; h > 0; h /= 2) {
         __syncthreads();
@@ -312,9 +301,9 @@ __global__ void __launch_bounds__(256) colsum_parts_kernel(const float* __restri
 }
 
 // Column sums of [parts, n] partial rows into out_g and out_b (+= when
-// acc_*; a null partial array skips its sum), in one launch.  As many columns
-// per workgroup as leave one workgroup per CU, so that few columns over many
-// partial rows still spread over the chip (a stage of 64-row sums in front
+// acc_*; a null partial array skips its sum), in one launch.  Few columns per
+// workgroup, or many row lanes, where there are few columns, so that they still
+// spread over the chip (as colsum_finalize_kernel; a stage of 64-row sums in front
 // cost a second dispatch: 8.5 -> 4.5 us at [256, 768] partials).
 int colsum_parts(const float* part_g, float* out_g, int acc_g, const float* part_b, float* out_b, int acc_b,
                  int64_t parts, int64_t n, const char* what) {
@@ -326,12 +315,12 @@ int colsum_parts(const float* part_g, float* out_g, int acc_g, const float* part
     if (!part_g) return WM_OK;
     const unsigned jobs = part_b ? 2u : 1u;
     const int64_t cols = n * jobs, want = num_cus();
-#define WM_CP(S)                                                                                              \
-    launch_kernel(colsum_parts_kernel<S>, dim3((unsigned)((n + S - 1) / S), 1u, jobs), dim3(256), 0, st, part_g, \
-                  part_b, parts, n, out_g, out_b, acc_g, acc_b)
-    if (cols >= 64 * want) WM_CP(64);
-    else if (cols >= 16 * want) WM_CP(16);
-    else WM_CP(4);
+#define WM_CP(S, NT)                                                                                          \
+    launch_kernel((colsum_parts_kernel<S, NT>), dim3((unsigned)((n + S - 1) / S), 1u, jobs), dim3(NT), 0, st, \
+                  part_g, part_b, parts, n, out_g, out_b, acc_g, acc_b)
+    if (cols >= 64 * want) WM_CP(64, 256);
+    else if (cols >= 8 * want) WM_CP(64, 1024);
+    else WM_CP(4, 256);
 #undef WM_CP
     return check_launch(what);
 }
