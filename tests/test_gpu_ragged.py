@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 from gpu_helpers import (_offset_dev, batchnorm_bwd, batchnorm_fwd, binary_bwd, binary_fwd, gemm,
-                         layernorm_bwd, layernorm_fwd, rng_normal, rng_uniform)
+                         layernorm_bwd, layernorm_fwd, reduce, rng_normal, rng_uniform)
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-5
@@ -181,3 +181,26 @@ def test_layernorm_row_lengths(wm, rows, n, accumulate):
         z = g0[k] if accumulate else np.float32(0)
         ok, w = oracle.close_scaled(got[k], ref[k] + z, scale[k] + np.abs(z), RTOL, 1e-30)
         assert ok, f"gradient {k} {w:.3g}x tolerance"
+
+
+# Strided reductions at the ends of the one-dispatch range (sixteen waves on up
+# to 320 or 512 positions) and just past it, below one position per wave, in
+# part-filled tiles of floats and float4s.
+@pytest.mark.parametrize("outer,n,inner", [(1, 129, 4), (1, 320, 10), (1, 321, 10), (3, 200, 64), (2, 130, 257),
+                                           (64, 197, 768), (140, 512, 3), (140, 513, 3), (130, 300, 36)])
+def test_strided_reductions_short_axis(wm, outer, n, inner):
+    x = np.rint(rng_normal((outer, n, inner), seed_of("red", outer, n, inner)) * 8).astype(np.float32) / 8  # ties
+    x[0, 0, 0] = np.nan  # a NaN wins only as the first element
+    x[0, n // 2, 1] = np.nan
+    x[-1, :, -1] = -np.inf
+    for op in ("max", "min", "argmax", "sum", "mean"):
+        y = np.nan_to_num(x, neginf=0.0) if op in ("sum", "mean") else x
+        v, i = reduce(op, y, outer, n, inner, want_idx=op in ("max", "min"))
+        if op in ("sum", "mean"):
+            ref, scale = (oracle.get(k).reduce(op, y, outer, n, inner)[0] for k in ("f64", "abs"))
+            ok, w = oracle.close_scaled(v, ref, scale, RTOL, 1e-30)
+            assert ok, f"{op} {w:.3g}x tolerance"
+        else:
+            rv, ri = oracle.get("f32").reduce(op, y, outer, n, inner)
+            assert oracle.bit_equal(v, rv), op
+            assert i is None or np.array_equal(i, ri), op

@@ -453,9 +453,9 @@ __global__ void __launch_bounds__(kBlock) reduce_rows_finalize_kernel(const floa
 
 // Lane l of each wave owns W adjacent inner positions (W = 4 with 128-bit
 // loads) of output row o, so a wave reads 64*W contiguous floats per position
-// of n.  The workgroup's 4 waves take four contiguous quarters of the chunk
-// [k0, k1) of n, each walking its quarter in increasing order with U loads
-// in flight; the four wave states are combined through LDS (sums in wave
+// of n.  The workgroup's waves take contiguous parts of the chunk
+// [k0, k1) of n, each walking its part in increasing order with U loads
+// in flight; the wave states are combined through LDS (sums in wave
 // order; the max family with 32-bit positions as chunk keys by an unsigned
 // maximum, with 64-bit positions by pairwise combines in wave order).
 // Items are (o, chunk, inner tile) triples, tile fastest; every thread of a
@@ -464,8 +464,12 @@ __global__ void __launch_bounds__(kBlock) reduce_rows_finalize_kernel(const floa
 // With K > 1 chunks the workgroup's state is a partial per column (a sum, or
 // the chunk key plus, for 64-bit positions, the position) that
 // reduce_cols_finalize_kernel combines.
-template <int OP, bool VEC, class I>
-__global__ void __launch_bounds__(kBlock) reduce_cols_kernel(const float* __restrict__ x, int64_t outer, int64_t n,
+//
+// NW = 16 waves instead of 4 where one chunk per column then fills the chip
+// well enough (launch_cols): the waves split n sixteen ways, and the second
+// pass, a dispatch of its own, is not needed.
+template <int OP, bool VEC, class I, int NW>
+__global__ void __launch_bounds__(NW * 64) reduce_cols_kernel(const float* __restrict__ x, int64_t outer, int64_t n,
                                                               int64_t inner, int64_t chunk, int64_t K,
                                                               float* __restrict__ val, int64_t* __restrict__ idx,
                                                               float* __restrict__ pv, uint64_t* __restrict__ pk,
@@ -473,7 +477,6 @@ __global__ void __launch_bounds__(kBlock) reduce_cols_kernel(const float* __rest
     constexpr int KIND = kind_of(OP);
     constexpr bool MX = KIND == 1;
     constexpr int W = VEC ? 4 : 1;
-    constexpr int NW = kBlock / 64;
     constexpr int U = VEC ? 8 : 4;
     constexpr bool KEYED = KIND != 0 && sizeof(I) == 4;  // states fold as chunk keys
     __shared__ float lv[KEYED ? 1 : NW][KEYED ? 1 : 64 * W];
@@ -487,7 +490,7 @@ __global__ void __launch_bounds__(kBlock) reduce_cols_kernel(const float* __rest
     const int64_t tiles = (inner + tile_elems - 1) / tile_elems;
     const int64_t items = outer * K * tiles;
 
-    // The four wave states (v, pos) -> wave 0 lanes hold the workgroup's
+    // The wave states (v, pos) -> wave 0 lanes hold the workgroup's
     // state of their W columns (sums, and the max family with 64-bit
     // positions).
     auto lds_combine = [&](float (&v)[W], I (&pos)[W]) {
@@ -503,7 +506,15 @@ __global__ void __launch_bounds__(kBlock) reduce_cols_kernel(const float* __rest
 #pragma unroll
                 for (int j = 0; j < W; ++j) {
                     if constexpr (KIND == 0) {
-                        v[j] = (lv[0][lane * W + j] + lv[1][lane * W + j]) + (lv[2][lane * W + j] + lv[3][lane * W + j]);
+                        float t[NW / 2];
+#pragma unroll
+                        for (int ww = 0; ww < NW / 2; ++ww)
+                            t[ww] = lv[2 * ww][lane * W + j] + lv[2 * ww + 1][lane * W + j];
+#pragma unroll
+                        for (int h = NW / 4; h > 0; h /= 2)
+#pragma unroll
+                            for (int ww = 0; ww < h; ++ww) t[ww] = t[2 * ww] + t[2 * ww + 1];
+                        v[j] = t[0];
                     } else {
                         v[j] = lv[0][lane * W + j];
                         pos[j] = li[0][lane * W + j];
@@ -515,7 +526,7 @@ __global__ void __launch_bounds__(kBlock) reduce_cols_kernel(const float* __rest
         }
     };
 
-    // The max family with 32-bit positions: the four wave states as chunk
+    // The max family with 32-bit positions: the wave states as chunk
     // keys, folded by an unsigned maximum (the keys' order is combine's
     // preference) -> wave 0 lanes hold the workgroup's keys of their W
     // columns.  Branch-free, where combine's NaN and emptiness tests cost
@@ -956,16 +967,26 @@ int launch_cols(const float* x, int64_t outer, int64_t n, int64_t inner, float* 
     if (outer * tiles < target_blocks)
         K = std::min<int64_t>((target_blocks + outer * tiles - 1) / (outer * tiles), (n + 127) / 128);
     K = std::max<int64_t>(std::min<int64_t>(K, 4096), 1);
+    // Where that asks for chunks of a short n, 16 waves on the whole of it (at
+    // most 20 positions each, 32 where half the CUs have a workgroup) spare the
+    // second dispatch.  Mean / max, both passes before and one now:
+    // [64, 197, 768] 15.8 / 15.7 -> 11.0 / 11.0 us, [197, 402, 3] 7.5 / 8.2 -> 5.4 /
+    // 6.0, [1, 300, 10] 5.1 / 6.1 -> 4.2 / 5.0; but [16, 512, 64] 7.8 / 8.2 against 8.5 /
+    // 11.4 and [1, 1000, 768] 8.9 / 9.2 against 20.8 / 22.0, which keep their chunks.
+    const bool tall = K > 1 && n <= (2 * outer * tiles >= num_cus() ? 512 : 320);
+    if (tall) K = 1;
     const int64_t chunk = (n + K - 1) / K;
     K = std::max<int64_t>(1, (n + chunk - 1) / chunk);
     std::unique_ptr<Partials> P;
     WM_TRY((take_partials<KIND, I>(K > 1 ? (size_t)(outer * K * inner) : 0, arena, P)));
     I* pi = static_cast<I*>(P->pi);
     dim3 grid(grid_for(outer * K * tiles, 1, 32));
-    if (vec) launch_kernel((reduce_cols_kernel<OP, true, I>), grid, dim3(kBlock), 0, st, x, outer, n, inner, chunk, K,
-                           val, idx, P->pv, P->pk, pi);
-    else launch_kernel((reduce_cols_kernel<OP, false, I>), grid, dim3(kBlock), 0, st, x, outer, n, inner, chunk, K,
-                       val, idx, P->pv, P->pk, pi);
+#define WM_COLS(V, NW)                                                                                             \
+    launch_kernel((reduce_cols_kernel<OP, V, I, NW>), grid, dim3(NW * 64), 0, st, x, outer, n, inner, chunk, K, val, \
+                  idx, P->pv, P->pk, pi)
+    if (tall) { if (vec) WM_COLS(true, 16); else WM_COLS(false, 16); }
+    else { if (vec) WM_COLS(true, 4); else WM_COLS(false, 4); }
+#undef WM_COLS
     WM_TRY(check_launch("wm_reduce(cols)"));
     if (K > 1) {
         launch_kernel((reduce_cols_finalize_kernel<OP, I>), dim3(grid_for(outer * inner, 16, 8)), dim3(kBlock), 0, st,
