@@ -204,3 +204,18 @@ def test_strided_reductions_short_axis(wm, outer, n, inner):
             rv, ri = oracle.get("f32").reduce(op, y, outer, n, inner)
             assert oracle.bit_equal(v, rv), op
             assert i is None or np.array_equal(i, ri), op
+
+
+# Broadcast forwards over rows of whole float4s that are not whole tiles, the
+# broadcast operand along the row, along the outer dims and both.
+@pytest.mark.parametrize("op", ["add", "div", "max"])
+@pytest.mark.parametrize("full,vec", [((5, 4), (5, 1)), ((3, 7, 12), (7, 1)), ((6, 5, 36), (1, 5, 1)), ((700, 64), (64,)),
+                                      ((9, 768), (9, 1)), ((2, 3, 5, 196), (3, 1, 196)), ((4, 6, 3136), (1, 6, 1)),
+                                      ((3, 2, 4, 2, 8), (2, 1, 2, 1)), ((2, 900), (1, 900)), ((33, 1028), (33, 1))])
+def test_broadcast_forward_ragged_rows(wm, op, full, vec):
+    s = seed_of(op, full, vec)
+    a, b = rng_normal(full, s), rng_uniform(vec, s + 1, 0.5, 2.0)
+    for x, y in ((a, b), (b, a)):
+        assert oracle.bit_equal(binary_fwd(op, x, y), oracle.get("f32").binary(op, x, y))
+    c, d = rng_normal(full[:-1] + (1,), s + 2), rng_uniform(full[-1:], s + 3, 0.5, 2.0)
+    assert oracle.bit_equal(binary_fwd(op, c, d), oracle.get("f32").binary(op, c, d))

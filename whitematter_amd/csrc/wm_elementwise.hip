@@ -404,6 +404,45 @@ __global__ void __launch_bounds__(kBlock, (rows_min_waves<OP, AI, BI, VEC, PAIRS
     }
 }
 
+// The same broadcast over a flat grid: thread i takes float4 i of the output
+// (inner % 4 == 0, aligned bases, fewer than 2^31 float4s) and finds its row by a
+// 32-bit division, so no lane is left over at the end of a row.  For rows that
+// are not whole 1024-element tiles: a channel bias over 56 x 56 planes (3136
+// elements, four tiles with the last 6 % full) takes 19.4 us against 29.0 for
+// binary_rows_kernel at [64, 64, 56, 56], over 14 x 14 planes 12.2 against 50.5
+// at [64, 512, 14, 14], and a row vector of 64 4.5 against 16.6 at [16384, 64].
+template <int OP, int AI, int BI>
+__global__ void __launch_bounds__(kBlock) binary_ragged_rows_kernel(float* __restrict__ out,
+                                                                     const float* __restrict__ a,
+                                                                     const float* __restrict__ b, uint32_t total4,
+                                                                     uint32_t inner4, RowDims d, int stream_a,
+                                                                     int stream_b) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= total4) return;
+    uint32_t row = i / inner4;
+    const int64_t c = (int64_t)(i - row * inner4) * 4;
+    int64_t oa = 0, ob = 0;
+    for (int k = d.nd - 1; k > 0; --k) {
+        const uint32_t s = (uint32_t)d.size[k], q = row / s, r = row - q * s;
+        oa += r * d.sa[k];
+        ob += r * d.sb[k];
+        row = q;
+    }
+    if (d.nd > 0) {
+        oa += row * d.sa[0];
+        ob += row * d.sb[0];
+    }
+    float4 va[1], vb[1], vr[1];
+    auto load = [&](const float* p, bool contiguous, int streamed) {
+        if (!contiguous) return make_float4(p[0], p[0], p[0], p[0]);
+        return streamed ? ld_stream(p + c) : *reinterpret_cast<const float4*>(p + c);
+    };
+    va[0] = load(a + oa, AI, stream_a);
+    vb[0] = load(b + ob, BI, stream_b);
+    binary_fwd_v<OP, 1>(vr, va, vb);
+    st_stream(out + 4 * (int64_t)i, vr[0]);
+}
+
 // Fallback for any collapsed layout: per-element index math over all dims.
 struct FullDims {
     int nd;
@@ -538,7 +577,37 @@ int launch_binary(float* out, const float* a, const float* b, const BcastLayout&
                            out, a, b, n4);
         return check_launch("wm_binary(flat)");
     }
-    if (inner >= 64 && (ia == 0 || ia == 1) && (ib == 0 || ib == 1)) {
+    const bool rows_ok = (ia == 0 || ia == 1) && (ib == 0 || ib == 1);
+    const bool vec_rows = (inner % 4) == 0 && aligned16(out) && aligned16(a) && aligned16(b);
+    // Rows that leave over an eighth of their 1024-element tiles empty (a
+    // quarter empty, [16384, 768], the two forms tie at 18.6-18.8 us; pow, bound
+    // by its arithmetic, keeps the tiles).
+    const int64_t row_tiles = (inner + 4 * kBlock - 1) / (4 * kBlock);
+    if (OP != WM_POW && rows_ok && vec_rows && nd > 1 && L.numel / 4 < ((int64_t)1 << 31) &&
+        8 * inner < 7 * row_tiles * 4 * kBlock) {
+        if constexpr (OP != WM_POW) {
+            RowDims d;
+            d.nd = nd - 1;
+            int stream_a = 0, stream_b = 0;
+            for (int i = 0; i < nd - 1; ++i) {
+                d.size[i] = L.size[i]; d.sa[i] = L.sa[i]; d.sb[i] = L.sb[i];
+                stream_a |= L.sa[i] != 0;
+                stream_b |= L.sb[i] != 0;
+            }
+            const uint32_t total4 = (uint32_t)(L.numel / 4);
+            const dim3 grid((total4 + kBlock - 1) / kBlock);
+#define WM_RAGGED(AI, BI)                                                                                   \
+    launch_kernel((binary_ragged_rows_kernel<OP, AI, BI>), grid, dim3(kBlock), 0, s, out, a, b, total4, \
+                  (uint32_t)(inner / 4), d, stream_a, stream_b)
+            if (ia && ib) WM_RAGGED(1, 1);
+            else if (ia) WM_RAGGED(1, 0);
+            else if (ib) WM_RAGGED(0, 1);
+            else WM_RAGGED(0, 0);
+#undef WM_RAGGED
+            return check_launch("wm_binary(ragged rows)");
+        }
+    }
+    if (inner >= 64 && rows_ok) {
         RowDims d;
         d.nd = nd - 1;
         int64_t rows = 1;
