@@ -96,6 +96,36 @@ def test_small_products(wm, m, n, k, batch, ta, tb):
         assert np.array_equal(got[..., n:], c0[..., n:])  # past the rows: untouched
 
 
+# Weight gradients x^T dY on the k split of the direct-to-LDS kernel: the lines of
+# its rule (18 and 200 tiles, k = 4096), equal slices and a shorter last one, and
+# sizes next to the lines that the library keeps.
+@pytest.mark.parametrize("m,n,k", [(384, 768, 4096), (768, 384, 4160), (640, 512, 6848), (2560, 1280, 4096),
+                                   (384, 768, 4032), (128, 2176, 4096), (1024, 1024, 4096), (384, 768, 4100)])
+@pytest.mark.parametrize("route", [0, 1])
+def test_long_weight_gradients(wm, m, n, k, route):
+    """alpha and accumulation, rows 4 past their end (NaN there), against float64
+    within 1e-5 of the sum of |terms|; the same bits again."""
+    r = np.random.default_rng(seed_of(m, n, k))
+    x, dy = np.full((k, m + 4), np.nan, np.float32), np.full((k, n + 4), np.nan, np.float32)
+    x[:, :m], dy[:, :n] = r.standard_normal((k, m), np.float32), r.standard_normal((k, n), np.float32)
+    c0 = r.standard_normal((m, n + 4), np.float32)
+    ref = x[:, :m].T.astype(np.float64) @ dy[:, :n]
+    scale = np.abs(x[:, :m].T).astype(np.float64) @ np.abs(dy[:, :n])
+    old = wm.lib().wm_gemm_library(-1)
+    wm.lib().wm_gemm_library(route)
+    try:
+        for acc in (0, 1):
+            got = [gemm(1, 0, m, n, k, 0.5, x.ravel(), m + 4, dy.ravel(), n + 4, c0.ravel(), n + 4, acc, None, 1, 1,
+                        None).reshape(c0.shape) for _ in range(2)]
+            base = c0[:, :n] if acc else 0.0
+            ok, w = oracle.close_scaled(got[0][:, :n], 0.5 * ref + base, 0.5 * scale + np.abs(base), RTOL)
+            assert ok, f"{w:.3g}x tolerance"
+            assert np.array_equal(got[0], got[1])
+            assert np.array_equal(got[0][:, n:], c0[:, n:])
+    finally:
+        wm.lib().wm_gemm_library(old)
+
+
 @pytest.mark.parametrize("offset", [0, 1, 2])
 @pytest.mark.parametrize("rows,cols", [(1, 1), (5, 3), (7, 4), (600, 13), (3, 127), (300, 255), (5, 1023), (4, 1024),
                                        (3, 1025), (2, 4099), (3, 32772), (2, 33001)])

@@ -470,7 +470,8 @@ __global__ void __launch_bounds__(kThreads) gemm_dma_kernel(GemmParams P) {
         aoff[u] = OpA::src(P.lda, m0, wave, lane, u);
         boff[u] = OpB::src(P.ldb, n0, wave, lane, u);
     }
-    const int nk = (int)(P.k / kDK);
+    // Of a k split (group = 1, problem = slice) the last slice may be shorter.
+    const int nk = (int)((P.kslices > 1 ? min(P.ksplit, P.k - (int64_t)blockIdx.y * P.ksplit) : P.k) / kDK);
     const uint32_t wofs = (uint32_t)__builtin_amdgcn_readfirstlane(wave) * 2048u;  // the wave's two blocks
     auto issue = [&](int64_t pp, int st, int bi) {  // stage st of problem pp into buffer bi
         const float* Ab = P.a + pp * P.sa0;
@@ -1206,7 +1207,7 @@ int64_t choose_kslices(int64_t work, int64_t k) {
 // contexts 45.7 / 64: two-level batches the library can only take as one
 // call per outer batch).  Batched products that gemm_dma_kernel takes run
 // there first (launch_gemm).  Unbatched products with m, n >= 128 and
-// k >= 256, and the other one-level batches of untransposed products with
+// k >= 256 (except the long-k weight gradients of split_beats_library), and the other one-level batches of untransposed products with
 // m, n >= 128, k <= 256, no bias and disjoint outputs, go to rocBLAS
 // (atomics off: the same bits on every run); the rest to gemm_kernel, and
 // while the library route is switched off (wm_gemm_library) every product
@@ -1311,13 +1312,17 @@ int try_library(bool ta, bool tb, const GemmParams& P) {
     return WM_OK;
 }
 
-// Whether gemm_dma_kernel takes P: one batch level, every tile interior (m,
-// n multiples of 128, k of 64), 16-byte rows, and no k split (gemm_kernel
-// splits k when few tiles meet a long k).
-bool dma_fits(bool vec, const GemmParams& P, int64_t tiles) {
+// Whether P is one gemm_dma_kernel can run: one batch level, every tile
+// interior (m, n multiples of 128, k of 64), 16-byte rows.
+bool dma_interior(bool vec, const GemmParams& P) {
     return vec && P.batch_inner == 1 && P.m % kTile == 0 && P.n % kTile == 0 && P.k > 0 &&
-           P.k % (4 * kDK) == 0 && P.c_aligned && P.ldc % 4 == 0 && (!P.bias || aligned16(P.bias)) &&
-           choose_kslices(tiles * P.batch, P.k) == 1;
+           P.k % (4 * kDK) == 0 && P.c_aligned && P.ldc % 4 == 0 && (!P.bias || aligned16(P.bias));
+}
+
+// Whether gemm_dma_kernel (or gemm_dma3_kernel) takes the whole of a batch's k
+// (few tiles with a long k are split).
+bool dma_fits(bool vec, const GemmParams& P, int64_t tiles) {
+    return dma_interior(vec, P) && choose_kslices(tiles * P.batch, P.k) == 1;
 }
 
 // gemm_dma_kernel for P, or 1 when the grid would not fit (the caller then
@@ -1342,6 +1347,54 @@ int launch_dma(bool ta, bool tb, GemmParams P, int64_t tiles) {
     else WM_DMA(true, true);
 #undef WM_DMA
     return check_launch("wm_gemm(dma)");
+}
+
+// The k split of an unbatched product on gemm_dma_kernel: slices of a whole
+// number of 64-k steps (the last may be shorter), as many as make the
+// estimated time least.  The workgroups are dealt out evenly, so the busiest
+// CU computes `rounds` slices, 4.0 us per step (5.0 when it has only one
+// workgroup, with nothing to cover its waits) and 3 us of set-up and epilogue
+// each; the second pass costs a dispatch and the partials' traffic.
+struct DmaSplit {
+    int64_t slices, steps;
+};
+
+DmaSplit choose_dma_split(const GemmParams& P, int64_t tiles) {
+    const int64_t total = P.k / (4 * kDK), cus = num_cus();
+    DmaSplit best{1, total};
+    double best_us = HUGE_VAL;
+    for (int64_t want = 1; want <= std::min<int64_t>(32, std::max<int64_t>(1, total / 4)); ++want) {
+        const int64_t steps = (total + want - 1) / want, slices = (total + steps - 1) / steps;
+        const int64_t rounds = (tiles * slices + cus - 1) / cus;
+        double us = (double)rounds * ((double)steps * (rounds == 1 ? 5.0 : 4.0) + 3.0);
+        if (slices > 1) us += 4.0 + (double)(P.m * P.n) * (double)(slices + 1) * 4.0 / 4e6;
+        if (us < best_us) {
+            best_us = us;
+            best = {slices, steps};
+        }
+    }
+    return best;
+}
+
+// Whether that beats the library on P, a weight gradient x^T dY over many
+// rows: k is long, and the output's 128 x 128 tiles alone do not fill the chip.
+// The library walks all of k in 64-256 wide tiles there and its rate depends
+// on how those happen to divide the chip: 16-149 TFLOP/s over 60 sizes
+// (m, n from 128 to 4096, k from 512 to 16320), where the split is at
+// 100-131.  Library / split, us: [768, 768] over 4096 62.6 / 59.6,
+// [768, 3072] over 4096 231.6 / 168.2, [1280, 640] over 4416 100.7 / 69.4,
+// [3072, 128] over 8768 420.7 / 75.6, [896, 768] over 10560 143.9 / 124.3,
+// [2048, 1152] over 6208 294.7 / 238.6; the two slower ones of 33 sizes inside
+// the lines are [1152, 896] over 14272 208.7 / 228.4 and [640, 2304] over
+// 9024 207.7 / 222.1.  Outside them the library keeps the product: fewer
+// than 18 tiles ([384, 384] over 6144 30.7 / 35.5), k below 4096 ([768, 1152]
+// over 1408 25.7 / 34.5, [896, 1024] over 3136 48.5 / 61.7), more than 200 tiles
+// ([2560, 1536] over 6400 355.4 / 394.2), and multiples of 64 tiles, which its
+// own tiles divide evenly ([1024, 1024] over 8192 125.4 / 137.9).  A Linear of
+// 4096 x 768 -> 3072, forward and backward, 546.5 -> 497.1 us; attention training
+// at [8, 512, 768] 965 -> 914 us.
+bool split_beats_library(bool ta, bool tb, const GemmParams& P, int64_t tiles) {
+    return ta && !tb && P.k >= 4096 && tiles >= 18 && tiles <= 200 && tiles % 64 != 0;
 }
 
 // Whether gemm_dma32_kernel takes P: A transposed, B not, n = 64 (one
@@ -1436,6 +1489,17 @@ int launch_small(SmallForm f, bool ta, bool tb, const GemmParams& P) {
     }
 }
 
+// The second pass of a k split: the slices' products [batch][kslices][m][n]
+// into F's C.
+int finish_split(const GemmParams& F, int kslices, const float* part) {
+    WM_TRY(check_launch("wm_gemm"));
+    const bool c_vec = F.c_aligned && (F.ldc & 3) == 0;
+    const int64_t items = F.batch * F.m * ((F.n + 3) / 4);
+    launch_kernel(splitk_reduce_kernel, dim3(grid_for(items, 256)), dim3(256), 0, stream(), part, kslices, F.m, F.n,
+                  F.batch, F.batch_inner, F.c, F.ldc, F.sc0, F.sc1, F.alpha, F.accumulate, F.bias, c_vec ? 1 : 0);
+    return check_launch("wm_gemm(split)");
+}
+
 int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
     GemmParams P = P0;
     // 64-wide column tiles for narrow products (attention's per-head products
@@ -1460,7 +1524,8 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
     // kernels.
     const bool routed = g_library.load(std::memory_order_relaxed) != 0;
     const int64_t work = tm * tn * P.batch;
-    const bool dma = dma_fits(vec, P, tm * tn) && (P.batch > 1 || !routed);
+    // Unbatched products of more than dma3's k take launch_gemm's split, below.
+    const bool dma = dma_fits(vec, P, tm * tn) && (P.batch > 1 || (!routed && P.k <= 256));
     const bool dma32 = narrow && dma32_fits(ta, tb, vec, P, tm * tn) && (P.batch > 1 || !routed);
     const bool lib_first = library_takes(ta, tb, P) && (P.batch == 1 || work >= num_cus());
     if (routed && P.k > 0 && !lib_first) {
@@ -1475,22 +1540,38 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
         const int r = launch_dma32(P, tm * tn);
         if (r != 1) return r;
     }
-    const int lib = try_library(ta, tb, P);
-    if (lib != 1) return lib;
+    const bool dma_split = P.batch == 1 && dma_interior(vec, P) &&
+                           (!routed || split_beats_library(ta, tb, P, tm * tn));
+    const DmaSplit split = dma_split ? choose_dma_split(P, tm * tn) : DmaSplit{1, 0};
+    if (!dma_split) {
+        const int lib = try_library(ta, tb, P);
+        if (lib != 1) return lib;
+    }
 
     // Split k: the partial products go to a workspace [batch][kslices][m][n]
     // (unscaled, overwritten), and a second pass adds them into C.
     int64_t kslices = choose_kslices(tm * tn * P.batch, P.k);
+    int64_t slice = P.k;
+    if (dma_split) {
+        kslices = split.slices;
+        slice = split.steps * 4 * kDK;
+    } else if (kslices > 1) {
+        slice = ((P.k + kslices - 1) / kslices + kBK - 1) / kBK * kBK;
+        kslices = (P.k + slice - 1) / slice;
+    }
     Workspace part(0);
     GemmParams F = P;  // the final C, for the second pass
+    P.ksplit = slice;
+    P.kslices = (int)kslices;
+    P.sck = 0;
     if (kslices > 1) {
-        const int64_t slice = ((P.k + kslices - 1) / kslices + kBK - 1) / kBK * kBK;
-        kslices = (P.k + slice - 1) / slice;
         const int64_t mn = P.m * P.n;
         part.p = ws_alloc((size_t)(P.batch * kslices * mn) * sizeof(float));
-        if (!part.p) return set_error(WM_ERR_NOMEM, "wm_gemm: split-k workspace");
-        P.ksplit = slice;
-        P.kslices = (int)kslices;
+        if (!part.p) {
+            // The library needs none.
+            const int lib = dma_split ? try_library(ta, tb, F) : 1;
+            return lib != 1 ? lib : set_error(WM_ERR_NOMEM, "wm_gemm: split-k workspace");
+        }
         P.c = part.as<float>();
         P.ldc = P.n;
         P.sc0 = P.batch_inner * kslices * mn;
@@ -1500,10 +1581,20 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
         P.accumulate = 0;
         P.bias = nullptr;
         P.c_aligned = (P.n & 3) == 0 ? 1 : 0;
-    } else {
-        P.ksplit = P.k;
-        P.kslices = 1;
-        P.sck = 0;
+    }
+    if (dma_split) {
+        // One problem per slice: the slices' starts are the batch strides.
+        P.batch = kslices;
+        P.sa0 = ta ? slice * P.lda : slice;
+        P.sb0 = tb ? slice : slice * P.ldb;
+        P.sc0 = P.m * P.n;
+        const dim3 g((unsigned)(tm * tn), (unsigned)kslices);
+        if (!ta && !tb) launch_kernel((gemm_dma_kernel<false, false>), g, dim3(kThreads), 0, s, P);
+        else if (!ta && tb) launch_kernel((gemm_dma_kernel<false, true>), g, dim3(kThreads), 0, s, P);
+        else if (ta && !tb) launch_kernel((gemm_dma_kernel<true, false>), g, dim3(kThreads), 0, s, P);
+        else launch_kernel((gemm_dma_kernel<true, true>), g, dim3(kThreads), 0, s, P);
+        if (kslices == 1) return check_launch("wm_gemm(dma)");
+        return finish_split(F, P.kslices, part.as<float>());
     }
     dim3 grid((unsigned)(tm * tn), (unsigned)std::min<int64_t>(P.batch * P.kslices, 65535));
 #define WM_GEMM(TA, TB, V)                                                                   \
@@ -1523,14 +1614,7 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
         else WM_GEMM(true, true, false);
     }
 #undef WM_GEMM
-    if (P.kslices > 1) {
-        WM_TRY(check_launch("wm_gemm"));
-        const bool c_vec = F.c_aligned && (F.ldc & 3) == 0;
-        const int64_t items = F.batch * F.m * ((F.n + 3) / 4);
-        launch_kernel(splitk_reduce_kernel, dim3(grid_for(items, 256)), dim3(256), 0, s, part.as<float>(),
-                           P.kslices, F.m, F.n, F.batch, F.batch_inner, F.c, F.ldc, F.sc0, F.sc1, F.alpha,
-                           F.accumulate, F.bias, c_vec ? 1 : 0);
-    }
+    if (P.kslices > 1) return finish_split(F, P.kslices, part.as<float>());
     return check_launch("wm_gemm");
 }
 
