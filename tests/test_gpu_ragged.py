@@ -249,3 +249,19 @@ def test_broadcast_forward_ragged_rows(wm, op, full, vec):
         assert oracle.bit_equal(binary_fwd(op, x, y), oracle.get("f32").binary(op, x, y))
     c, d = rng_normal(full[:-1] + (1,), s + 2), rng_uniform(full[-1:], s + 3, 0.5, 2.0)
     assert oracle.bit_equal(binary_fwd(op, c, d), oracle.get("f32").binary(op, c, d))
+
+
+# Column sums of row vectors at the lines of their second pass: 4 and 64
+# columns per workgroup, a thread per column, and a partial last tile.
+@pytest.mark.parametrize("rows,cols", [(37, 2044), (37, 2048), (9, 16380), (9, 16384), (3, 65532), (5, 65536),
+                                       (70, 65540), (2, 300004)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_wide_row_vector_gradient(wm, rows, cols, accumulate):
+    """Small whole numbers: every sum is exact in float32."""
+    r = np.random.default_rng(seed_of("wide", rows, cols))
+    g = r.integers(-8, 9, (rows, cols)).astype(np.float32)
+    a, b = np.ones((rows, cols), np.float32), np.ones((cols,), np.float32)
+    b0 = r.integers(-8, 9, (cols,)).astype(np.float32) if accumulate else None
+    ga, gb = binary_bwd("add", g, a, b, None, None, b0)
+    assert np.array_equal(ga, g)
+    assert np.array_equal(gb, g.sum(0) + (b0 if accumulate else 0.0))

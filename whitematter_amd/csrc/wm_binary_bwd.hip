@@ -192,26 +192,32 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
 // ~256 workgroups (64 columns left 16 workgroups each walking 256 rows per
 // wave: 13.6 us); from 2048 columns on, 64 columns with 16 groups read whole
 // lines with as many rows in flight ([512, 4096] partials 5.2 us against 11.5
-// for 16 columns with 16 groups).
+// for 16 columns with 16 groups); at most 8 partial rows of 65536 columns or
+// more, a thread per column (a row vector's gradient over [2, 500000] 9.8 us
+// with 64 columns and their tree, 7.4 so; [4, 2^20] 19.3 and 14.2; with 32
+// partial rows the tree is 1 us faster).
 template <int S, int NT>
 __global__ void __launch_bounds__(NT) colsum_finalize_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                                   int acc, int64_t K, int64_t C, int64_t O) {
     constexpr int G = NT / S;
     __shared__ float lds[G][S];
     const int cl = threadIdx.x % S, g = threadIdx.x / S;
+    const int64_t tiles = (C + S - 1) / S;
     for (int64_t ou = blockIdx.y; ou < O; ou += gridDim.y) {
-        const int64_t c = (int64_t)blockIdx.x * S + cl;
-        lds[g][cl] = c < C ? strided_sum<G>(part + ou * K * C + c, C, g, K) : 0.f;
+        for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+            const int64_t c = tile * S + cl;
+            lds[g][cl] = c < C ? strided_sum<G>(part + ou * K * C + c, C, g, K) : 0.f;
 #pragma unroll
-        for (int h = G / 2; h > 0; h /= 2) {
+            for (int h = G / 2; h > 0; h /= 2) {
+                __syncthreads();
+                if (g < h) lds[g][cl] += lds[g + h][cl];
+            }
+            if (g == 0 && c < C) {
+                float* dst = out + ou * C + c;
+                *dst = acc ? *dst + lds[0][cl] : lds[0][cl];
+            }
             __syncthreads();
-            if (g < h) lds[g][cl] += lds[g + h][cl];
         }
-        if (g == 0 && c < C) {
-            float* dst = out + ou * C + c;
-            *dst = acc ? *dst + lds[0][cl] : lds[0][cl];
-        }
-        __syncthreads();
     }
 }
 
@@ -220,9 +226,10 @@ int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, in
     const int64_t want = (int64_t)num_cus(), cols = C * O;
 #define WM_CF(S, NT)                                                                                      \
     launch_kernel((colsum_finalize_kernel<S, NT>),                                                        \
-                  dim3((unsigned)((C + S - 1) / S), (unsigned)std::min<int64_t>(O, 65535)), dim3(NT), 0, st, part, \
-                  out, acc, K, C, O)
-    if (cols >= 64 * want) WM_CF(64, kBlock);
+                  dim3((unsigned)std::min<int64_t>((C + S - 1) / S, 1 << 20), (unsigned)std::min<int64_t>(O, 65535)), \
+                  dim3(NT), 0, st, part, out, acc, K, C, O)
+    if (cols >= 256 * want && K <= 8) WM_CF(256, kBlock);
+    else if (cols >= 64 * want) WM_CF(64, kBlock);
     else if (cols >= 8 * want) WM_CF(64, 1024);
     else WM_CF(4, kBlock);
 #undef WM_CF
