@@ -265,3 +265,55 @@ def test_wide_row_vector_gradient(wm, rows, cols, accumulate):
     ga, gb = binary_bwd("add", g, a, b, None, None, b0)
     assert np.array_equal(ga, g)
     assert np.array_equal(gb, g.sum(0) + (b0 if accumulate else 0.0))
+
+
+# Many [R, C] problems sharing workgroups: rows of one unit up to more than a
+# wave, one to a few rows each (a row lane per row, and several rows per lane
+# where there is enough work), a partial last group of problems, more groups
+# than a grid's z, and few long rows (tiles of 128 and 256 units).
+MANY_SHAPES = [((3, 2, 1), (3, 1, 1)), ((300, 2, 8), (300, 1, 8)), ((70, 3, 7), (70, 1, 7)), ((1001, 5, 4), (1001, 1, 4)),
+               ((130, 2, 130), (130, 1, 130)), ((9000, 3, 33), (9000, 1, 33)), ((70000, 2, 3), (70000, 1, 3)),
+               ((33, 6, 260), (33, 1, 260)), ((2, 300001), (300001,)), ((3, 4098), (4098,)), ((90, 9, 3, 64), (90, 1, 3, 64))]
+
+
+@pytest.mark.parametrize("op", ["add", "div", "pow"])
+@pytest.mark.parametrize("full,vec", MANY_SHAPES)
+def test_broadcast_backward_many_small_problems(wm, op, full, vec):
+    test_broadcast_backward_edges(wm, op, full, vec)
+
+
+def kernel_ms(wm, call, reps=12):
+    """The kernels' time of one call, the least of `reps`."""
+    best = C.c_float()
+    ms = []
+    for _ in range(reps):
+        wm.call("wm_span_begin")
+        call()
+        wm.call("wm_span_end", C.byref(best), None, None)
+        ms.append(best.value)
+    return min(ms)
+
+
+def pace(wm, nbytes, call):
+    """How many times longer than a copy of `nbytes` (read and written) a call
+    takes."""
+    n = nbytes // 32 * 4
+    src, dst = wm.DeviceArray((n,)), wm.DeviceArray((n,))
+    src.fill(1.0)
+    return kernel_ms(wm, call) / kernel_ms(wm, lambda: wm.call("wm_copy_kernel", dst.vp, src.vp, n))
+
+
+def backward_pace(wm, full, vec):
+    """pace() of the add backward of two device tensors of ones."""
+    g, a, b = (wm.DeviceArray(s) for s in (full, full, vec))
+    ga, gb = wm.DeviceArray(full), wm.DeviceArray(vec)
+    for d in (g, a, b):
+        d.fill(1.0)
+    return pace(wm, 8 * g.size + 4 * b.size, lambda: wm.binary_bwd(wm.ADD, g, a, b, None, ga, False, gb, False))
+
+
+# Over [2^20, 2, 4] a workgroup per problem took a hundred times a copy.
+@pytest.mark.parametrize("full,vec", [((1 << 20, 2, 4), (1 << 20, 1, 4)), ((65536, 3, 7), (65536, 1, 7)),
+                                      ((2, 4000001), (1, 4000001))])
+def test_broadcast_backward_pace(wm, full, vec):
+    assert backward_pace(wm, full, vec) < 5.0

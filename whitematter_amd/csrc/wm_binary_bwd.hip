@@ -479,29 +479,43 @@ __global__ void __launch_bounds__(kBlock) rowsum_finalize_kernel(const float* __
 // ---------------------------------------------------------------------------
 
 // A unit is a float4 (VEC: C % 4 == 0 and aligned bases) or a float.  A
-// workgroup takes `tu` adjacent units of one column tile and 256 / tu rows at
-// a time, so a short row (a ten-class bias, a 64-wide feature) still fills
-// its waves; row groups are handed out cyclically as in bwd_colsum_kernel.
-// The workgroup's row lanes are added through LDS in a fixed tree, then the
-// column sums go to the gradient (one row group) or to its partials.
+// workgroup takes `tu` adjacent units of one column tile, `rl` rows at a
+// time, of `no` adjacent o, so a short row (a ten-class bias, a 64-wide
+// feature) still fills its waves, and so do many o of a few short rows; row
+// groups are handed out cyclically as in bwd_colsum_kernel.  The row lanes of
+// an o are added through LDS in a fixed tree, then the column sums go to the
+// gradient (one row group) or to its partials.
 //
-// Bound by latency at small sizes (each thread keeps kColRows rows in
+// Bound by latency at small sizes (each thread keeps col_rows() rows in
 // flight) and by HBM at large ones.  Before, every such layout except
 // [R, C] with C % 4 == 0 ran one thread per column over all R rows: a bias
 // gradient over [5912, 30] took 2441 us and one over [4, 27, 3616] with a
 // [4, 1, 3616] operand 16 us; rows of fewer than 1024 floats left lanes idle.
-template <int OP>
-constexpr int col_rows() { return OP == WM_POW || OP == WM_DIV ? 1 : 4; }
+template <int OP, bool VEC>
+constexpr int col_rows() { return OP == WM_POW ? (VEC ? 1 : 2) : VEC && OP == WM_DIV ? 1 : 4; }
+
+// A dimension of a launch has fewer than 2^32 threads.
+constexpr int64_t kMaxGrid = ((int64_t)1 << 32) / kBlock - 1;
+
+struct ColTile {
+    int tu, rl, no;
+    float inv_tu, inv_rl;
+    int64_t tiles, groups, K;  // column tiles, o groups, row groups
+};
+
+// Waves per SIMD to compile for (pow over float4s would go to 3: 27.5 us
+// against 24.9 at [4096, 4, 256]).
+template <int OP, bool VEC>
+constexpr int col_min_waves() { return OP == WM_POW && VEC ? 4 : 1; }
 
 template <int OP, bool VB, bool VEC>
-__global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restrict__ g, const float* __restrict__ F,
-                                                           const float* __restrict__ V, const float* __restrict__ o,
-                                                           float* __restrict__ gF, int accF, float* __restrict__ gV,
-                                                           int accV, float* __restrict__ part, int64_t O, int64_t R,
-                                                           int64_t C, int tu) {
+__global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_kernel(
+    const float* __restrict__ g, const float* __restrict__ F, const float* __restrict__ V,
+    const float* __restrict__ o, float* __restrict__ gF, int accF, float* __restrict__ gV, int accV,
+    float* __restrict__ part, int64_t O, int64_t R, int64_t C, ColTile t) {
     binary_prologue<OP>();
     constexpr int WD = VEC ? 4 : 1;
-    constexpr int UR = col_rows<OP>();
+    constexpr int UR = col_rows<OP, VEC>();
     __shared__ float lds[kBlock][WD];
     const bool want_v = gV != nullptr;
     const bool gF_reads_F = VB ? da_reads_a<OP>() : db_reads_b<OP>();
@@ -512,11 +526,14 @@ __global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restric
     const bool need_o = want_o && o;
     const bool need_F = (gF && gF_reads_F) || (want_v && gV_reads_F) || (want_o && !o);
     const bool need_V = (gF && gF_reads_V) || (want_v && gV_reads_V) || (want_o && !o);
-    const int rb = kBlock / tu;
-    const int tr = (int)threadIdx.x / tu, tc = (int)threadIdx.x - tr * tu;
+    const int tu = t.tu, rl = t.rl, no = t.no;
+    // x / y of x < 256 (exact: the quotient's distance from a whole number is
+    // at least 0.5 / y).
+    auto quot = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
+    const int tq = quot((int)threadIdx.x, t.inv_tu), tc = (int)threadIdx.x - tq * tu;
+    const int so = quot(tq, t.inv_rl), tr = tq - so * rl;  // this thread's o and row lane
     const int64_t c = ((int64_t)blockIdx.x * tu + tc) * WD;
-    const bool live = tr < rb && c < C;
-    const int64_t K = gridDim.y, step = K * rb;
+    const int64_t K = gridDim.y, step = K * rl;
     auto load = [](const float* p, float(&v)[WD]) {
         if constexpr (VEC) {
             const float4 q = ld_stream(p);
@@ -525,7 +542,9 @@ __global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restric
             v[0] = ld_stream1(p);
         }
     };
-    for (int64_t ou = blockIdx.z; ou < O; ou += gridDim.z) {
+    for (int64_t ob = (int64_t)blockIdx.z * no; ob < O; ob += (int64_t)gridDim.z * no) {
+        const int64_t ou = ob + so;
+        const bool live = so < no && ou < O && c < C;
         const int64_t base = ou * R * C + c;
         float s[WD], vv[WD];
 #pragma unroll
@@ -534,7 +553,7 @@ __global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restric
 #pragma unroll
             for (int j = 0; j < WD; ++j) vv[j] = V[ou * C + c + j];
         }
-        for (int64_t r0 = (int64_t)blockIdx.y * rb + tr; live && r0 < R; r0 += step * UR) {
+        for (int64_t r0 = (int64_t)blockIdx.y * rl + tr; live && r0 < R; r0 += step * UR) {
             float vg[UR][WD], vf[UR][WD], vo[UR][WD], old[UR][WD];
 #pragma unroll
             for (int u = 0; u < UR; ++u) {
@@ -572,13 +591,13 @@ __global__ void __launch_bounds__(kBlock) bwd_cols_kernel(const float* __restric
             }
         }
         if (!want_v) continue;
-        if (rb > 1) {
+        if (rl > 1) {
 #pragma unroll
             for (int j = 0; j < WD; ++j) lds[threadIdx.x][j] = s[j];
-            for (int n = rb; n > 1;) {
+            for (int n = rl; n > 1;) {
                 const int h = (n + 1) / 2;
                 __syncthreads();
-                if (tr + h < n) {
+                if (so < no && tr + h < n) {
 #pragma unroll
                     for (int j = 0; j < WD; ++j) lds[threadIdx.x][j] += lds[threadIdx.x + h * tu][j];
                 }
@@ -764,27 +783,48 @@ __global__ void __launch_bounds__(kBlock) bwd_generic_kernel(const float* __rest
 // Host dispatch
 // ---------------------------------------------------------------------------
 
-// [O, R, C] with V [O, 1, C].  64 adjacent units per row and workgroup (a
-// contiguous 1 KB of float4s), fewer when a row is shorter, so small R still
-// spreads over the row lanes; row groups until ~1024 workgroups run.  A group
-// of at most 4 steps of a workgroup is not split: its steps cost less than
-// the ~4 us of the second dispatch that adds the groups' partials.
+// The tile of bwd_cols_kernel for R rows of `units` units and O problems (see
+// there).  Row lanes: a row each while ~1024 workgroups would not fill, up to
+// col_rows() rows each (`most`) beyond; then as many adjacent units as the row
+// lanes leave, at least 64 (a contiguous 1 KB of float4s), and as many o as
+// fit.  Row groups until ~1024 workgroups run; a group of at most 4 steps of a
+// workgroup is not split: its steps cost less than the ~4 us of the second
+// dispatch that adds the groups' partials.
+//
+// One o per workgroup and 256 / tu row lanes whatever R left most lanes idle
+// at small R (and one thread per column, before, all but the first of each
+// row's floats uncoalesced): add over [65536, 2, 8] with [65536, 1, 8] 16.7 us
+// per column, 127.6 per o, 6.2 so; [2^20, 2, 4] 99.5, 1664 and 25.5; [16384, 2,
+// 256] 99.4, 36.6 and 18.5; a row vector over [2, 4000001] 69.5, 82.2 and 30.5.
+ColTile col_tile(int64_t O, int64_t R, int64_t units, int most) {
+    ColTile t;
+    const int64_t rows = std::max<int64_t>(1, std::min<int64_t>(most, O * R * units / (1024 * kBlock)));
+    const int64_t lanes = std::min<int64_t>(kBlock, (R + rows - 1) / rows);
+    const int64_t tu = std::min<int64_t>(units, std::max<int64_t>(64, kBlock / lanes));
+    const int64_t rb = kBlock / tu;
+    t.tu = (int)tu;
+    t.rl = (int)std::min(rb, lanes);
+    t.no = (int)std::min<int64_t>(O, rb / t.rl);
+    t.inv_tu = 1.0f / (float)t.tu;
+    t.inv_rl = 1.0f / (float)t.rl;
+    t.tiles = (units + tu - 1) / tu;
+    t.groups = (O + t.no - 1) / t.no;
+    const int64_t steps = (R + (int64_t)t.rl * most - 1) / ((int64_t)t.rl * most), wgs = t.tiles * t.groups;
+    t.K = steps > 4 && wgs < 1024 ? std::min<int64_t>(steps, (1024 + wgs - 1) / wgs) : 1;
+    return t;
+}
+
 template <int OP>
-int launch_cols(bool vb, bool vec, const float* g, const float* F, const float* V, const float* o, float* gF, int accF,
-                float* gV, int accV, int64_t O, int64_t R, int64_t C) {
+int launch_cols(const ColTile& t, bool vb, bool vec, const float* g, const float* F, const float* V, const float* o,
+                float* gF, int accF, float* gV, int accV, int64_t O, int64_t R, int64_t C) {
     hipStream_t st = stream();
-    const int64_t units = vec ? C / 4 : C;
-    const int tu = (int)std::min<int64_t>(units, 64);
-    const int64_t tiles = (units + tu - 1) / tu;
-    const int64_t steps = (R + (int64_t)(kBlock / tu) * col_rows<OP>() - 1) / ((int64_t)(kBlock / tu) * col_rows<OP>());
-    int64_t K = 1;
-    if (steps > 4 && tiles * O < 1024) K = std::min<int64_t>(steps, (1024 + tiles * O - 1) / (tiles * O));
+    const int64_t K = t.K;
     Workspace ws(gV && K > 1 ? (size_t)(O * K * C) * sizeof(float) : 0);
     if (gV && K > 1 && !ws.p) return set_error(WM_ERR_NOMEM, "wm_binary_bwd: workspace");
-    const dim3 grid((unsigned)tiles, (unsigned)K, (unsigned)std::min<int64_t>(O, 65535));
-#define WM_BC(VBv, VECv)                                                                                          \
-    launch_kernel((bwd_cols_kernel<OP, VBv, VECv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV, accV,    \
-                  ws.as<float>(), O, R, C, tu)
+    const dim3 grid((unsigned)t.tiles, (unsigned)K, (unsigned)std::min<int64_t>(t.groups, 65535));
+#define WM_BC(VBv, VECv)                                                                                       \
+    launch_kernel((bwd_cols_kernel<OP, VBv, VECv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV, accV, \
+                  ws.as<float>(), O, R, C, t)
     if (vb) { if (vec) WM_BC(true, true); else WM_BC(true, false); }
     else { if (vec) WM_BC(false, true); else WM_BC(false, false); }
 #undef WM_BC
@@ -865,8 +905,10 @@ int launch_binary_bwd(const float* g, const float* a, const float* b, const floa
             const int64_t O = nd == 3 ? size[0] : 1, R = size[nd - 2];
             // bwd_colsum_kernel keeps the wide aligned [R, C] it was shaped
             // for (one row per step, 1024-column tiles).
-            if (!(O == 1 && vec && C >= kBlock * 4))
-                return launch_cols<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, O, R, C);
+            const ColTile t = vec ? col_tile(O, R, C / 4, col_rows<OP, true>())
+                                  : col_tile(O, R, C, col_rows<OP, false>());
+            if (!(O == 1 && vec && C >= kBlock * 4) && t.tiles <= kMaxGrid)
+                return launch_cols<OP>(t, vb, vec, g, F, V, o, gF, accF, gV, accV, O, R, C);
         } else if (nd == 3 && sv[0] == 0 && sv[1] == 1 && sv[2] == 0) {
             return launch_channel<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, size[0], size[1], C);
         }
