@@ -282,6 +282,38 @@ def test_broadcast_backward_many_small_problems(wm, op, full, vec):
     test_broadcast_backward_edges(wm, op, full, vec)
 
 
+# Many channels of a few elements sharing workgroups: planes of 1 to 32 units
+# (the longest whose channels share them) and one more, of floats and of
+# float4s, one and several row groups, a partial last tile; just fewer channels
+# than share them.
+CHANNEL_SHAPES = [((2, 4096, 4), (4096, 1)), ((3, 4099, 3), (4099, 1)), ((2, 4100, 31), (4100, 1)),
+                  ((3, 4096, 32), (4096, 1)), ((2, 4097, 33), (4097, 1)), ((2, 4098, 128), (4098, 1)),
+                  ((2, 4098, 132), (4098, 1)), ((70, 4096, 2), (4096, 1)), ((9, 5000, 4, 4), (5000, 1, 1)),
+                  ((300, 4101, 1, 2), (4101, 1, 1)), ((3, 4095, 3), (4095, 1))]
+
+
+@pytest.mark.parametrize("op", ["add", "div", "pow"])
+@pytest.mark.parametrize("full,vec", CHANNEL_SHAPES)
+def test_broadcast_backward_many_channels(wm, op, full, vec):
+    test_broadcast_backward_edges(wm, op, full, vec)
+
+
+def test_broadcast_backward_channel_count(wm):
+    """More channels than a workgroup each could be launched for (2^32 threads):
+    ones, so every channel's sum is its element count."""
+    k = (1 << 24) + 3
+    full, vec = (2, k, 2), (k, 1)
+    g, a, b = (wm.DeviceArray(s) for s in (full, full, vec))
+    ga, gb = wm.DeviceArray(full), wm.DeviceArray(vec)
+    for d in (g, a, b):
+        d.fill(1.0)
+    ga.fill(np.nan)
+    gb.fill(np.nan)
+    wm.binary_bwd(wm.ADD, g, a, b, None, ga, False, gb, False)
+    assert np.all(gb.to_host() == 2.0 * full[2])
+    assert np.all(ga.to_host() == 1.0)
+
+
 def kernel_ms(wm, call, reps=12):
     """The kernels' time of one call, the least of `reps`."""
     best = C.c_float()
@@ -312,8 +344,10 @@ def backward_pace(wm, full, vec):
     return pace(wm, 8 * g.size + 4 * b.size, lambda: wm.binary_bwd(wm.ADD, g, a, b, None, ga, False, gb, False))
 
 
-# Over [2^20, 2, 4] a workgroup per problem took a hundred times a copy.
+# A workgroup per problem or channel took 21 to 142 times a copy over these, a
+# row vector over two long rows 6.7.
 @pytest.mark.parametrize("full,vec", [((1 << 20, 2, 4), (1 << 20, 1, 4)), ((65536, 3, 7), (65536, 1, 7)),
-                                      ((2, 4000001), (1, 4000001))])
+                                      ((2, 4000001), (1, 4000001)), ((2, 1 << 20, 2), (1, 1 << 20, 1)),
+                                      ((4, 200000, 3), (1, 200000, 1))])
 def test_broadcast_backward_pace(wm, full, vec):
     assert backward_pace(wm, full, vec) < 5.0

@@ -475,7 +475,8 @@ __global__ void __launch_bounds__(kBlock) rowsum_finalize_kernel(const float* __
 }
 
 // ---------------------------------------------------------------------------
-// cols: F full [O,R,C], V [O,1,C] (O = 1: a row vector), any C
+// cols: F full [O,R,C], V [O,1,C] (O = 1: a row vector), any C; and
+// [R,K,I] with V [1,K,1], many channels of a few elements
 // ---------------------------------------------------------------------------
 
 // A unit is a float4 (VEC: C % 4 == 0 and aligned bases) or a float.  A
@@ -484,7 +485,8 @@ __global__ void __launch_bounds__(kBlock) rowsum_finalize_kernel(const float* __
 // feature) still fills its waves, and so do many o of a few short rows; row
 // groups are handed out cyclically as in bwd_colsum_kernel.  The row lanes of
 // an o are added through LDS in a fixed tree, then the column sums go to the
-// gradient (one row group) or to its partials.
+// gradient (one row group) or to its partials.  With fold > 0 (O = 1), V has
+// an element per `fold` adjacent units, whose column sums are added in order.
 //
 // Bound by latency at small sizes (each thread keeps col_rows() rows in
 // flight) and by HBM at large ones.  Before, every such layout except
@@ -498,7 +500,7 @@ constexpr int col_rows() { return OP == WM_POW ? (VEC ? 1 : 2) : VEC && OP == WM
 constexpr int64_t kMaxGrid = ((int64_t)1 << 32) / kBlock - 1;
 
 struct ColTile {
-    int tu, rl, no;
+    int tu, rl, no, fold;
     float inv_tu, inv_rl;
     int64_t tiles, groups, K;  // column tiles, o groups, row groups
 };
@@ -508,7 +510,7 @@ struct ColTile {
 template <int OP, bool VEC>
 constexpr int col_min_waves() { return OP == WM_POW && VEC ? 4 : 1; }
 
-template <int OP, bool VB, bool VEC>
+template <int OP, bool VB, bool VEC, bool FOLD>
 __global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_kernel(
     const float* __restrict__ g, const float* __restrict__ F, const float* __restrict__ V,
     const float* __restrict__ o, float* __restrict__ gF, int accF, float* __restrict__ gV, int accV,
@@ -526,13 +528,14 @@ __global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_k
     const bool need_o = want_o && o;
     const bool need_F = (gF && gF_reads_F) || (want_v && gV_reads_F) || (want_o && !o);
     const bool need_V = (gF && gF_reads_V) || (want_v && gV_reads_V) || (want_o && !o);
-    const int tu = t.tu, rl = t.rl, no = t.no;
+    const int tu = t.tu, rl = t.rl, no = t.no, fold = FOLD ? t.fold : 1;
     // x / y of x < 256 (exact: the quotient's distance from a whole number is
     // at least 0.5 / y).
     auto quot = [](int x, float inv) { return (int)(((float)x + 0.5f) * inv); };
     const int tq = quot((int)threadIdx.x, t.inv_tu), tc = (int)threadIdx.x - tq * tu;
     const int so = quot(tq, t.inv_rl), tr = tq - so * rl;  // this thread's o and row lane
     const int64_t c = ((int64_t)blockIdx.x * tu + tc) * WD;
+    const int64_t ch = FOLD ? c / (WD * fold) : 0;
     const int64_t K = gridDim.y, step = K * rl;
     auto load = [](const float* p, float(&v)[WD]) {
         if constexpr (VEC) {
@@ -551,7 +554,7 @@ __global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_k
         for (int j = 0; j < WD; ++j) s[j] = vv[j] = 0.f;
         if (live && need_V) {
 #pragma unroll
-            for (int j = 0; j < WD; ++j) vv[j] = V[ou * C + c + j];
+            for (int j = 0; j < WD; ++j) vv[j] = V[FOLD ? ch : ou * C + c + j];
         }
         for (int64_t r0 = (int64_t)blockIdx.y * rl + tr; live && r0 < R; r0 += step * UR) {
             float vg[UR][WD], vf[UR][WD], vo[UR][WD], old[UR][WD];
@@ -605,7 +608,19 @@ __global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_k
             }
 #pragma unroll
             for (int j = 0; j < WD; ++j) s[j] = lds[threadIdx.x][j];
-            __syncthreads();  // the next o writes LDS again
+            __syncthreads();  // LDS is written again: by the next o, or below
+        }
+        if constexpr (FOLD) {
+            float sum = s[0];
+            if constexpr (VEC) sum = (s[0] + s[1]) + (s[2] + s[3]);
+            lds[threadIdx.x][0] = sum;
+            __syncthreads();
+            if (tr == 0 && live && c == ch * (WD * fold)) {
+                for (int f = 1; f < fold; ++f) sum += lds[threadIdx.x + f][0];
+                if (K == 1) gV[ch] = accV ? gV[ch] + sum : sum;
+                else part[blockIdx.y * (C / (WD * fold)) + ch] = sum;
+            }
+            continue;  // O = 1: no LDS write follows
         }
         if (tr == 0 && live) {
 #pragma unroll
@@ -629,7 +644,7 @@ __global__ void __launch_bounds__(kBlock, (col_min_waves<OP, VEC>())) bwd_cols_k
 // channel k's O * I / W units (W = 4: I % 4 == 0 and aligned bases), 256
 // adjacent units at a time across plane ends, so every lane has work at any
 // plane size; the position advances by the constant (256 / U planes, 256 % U
-// units) without dividing.  kChanUnits steps' loads are in flight per
+// units) without dividing.  chan_units() steps' loads are in flight per
 // thread.  The workgroups running at one time take the same planes of
 // neighbouring channels, which lie side by side in memory.  HBM-bound; one
 // thread per channel summing it element by element took 77.4 ms at
@@ -796,15 +811,17 @@ __global__ void __launch_bounds__(kBlock) bwd_generic_kernel(const float* __rest
 // row's floats uncoalesced): add over [65536, 2, 8] with [65536, 1, 8] 16.7 us
 // per column, 127.6 per o, 6.2 so; [2^20, 2, 4] 99.5, 1664 and 25.5; [16384, 2,
 // 256] 99.4, 36.6 and 18.5; a row vector over [2, 4000001] 69.5, 82.2 and 30.5.
-ColTile col_tile(int64_t O, int64_t R, int64_t units, int most) {
+ColTile col_tile(int64_t O, int64_t R, int64_t units, int most, int fold) {
     ColTile t;
     const int64_t rows = std::max<int64_t>(1, std::min<int64_t>(most, O * R * units / (1024 * kBlock)));
     const int64_t lanes = std::min<int64_t>(kBlock, (R + rows - 1) / rows);
-    const int64_t tu = std::min<int64_t>(units, std::max<int64_t>(64, kBlock / lanes));
+    int64_t tu = std::min<int64_t>(units, std::max<int64_t>(64, kBlock / lanes));
+    if (fold) tu -= tu % fold;  // fold <= 64
     const int64_t rb = kBlock / tu;
     t.tu = (int)tu;
     t.rl = (int)std::min(rb, lanes);
     t.no = (int)std::min<int64_t>(O, rb / t.rl);
+    t.fold = fold;
     t.inv_tu = 1.0f / (float)t.tu;
     t.inv_rl = 1.0f / (float)t.rl;
     t.tiles = (units + tu - 1) / tu;
@@ -818,18 +835,23 @@ template <int OP>
 int launch_cols(const ColTile& t, bool vb, bool vec, const float* g, const float* F, const float* V, const float* o,
                 float* gF, int accF, float* gV, int accV, int64_t O, int64_t R, int64_t C) {
     hipStream_t st = stream();
-    const int64_t K = t.K;
-    Workspace ws(gV && K > 1 ? (size_t)(O * K * C) * sizeof(float) : 0);
+    const int64_t K = t.K, nv = t.fold ? C / ((vec ? 4 : 1) * t.fold) : C;  // V's elements per o
+    Workspace ws(gV && K > 1 ? (size_t)(O * K * nv) * sizeof(float) : 0);
     if (gV && K > 1 && !ws.p) return set_error(WM_ERR_NOMEM, "wm_binary_bwd: workspace");
     const dim3 grid((unsigned)t.tiles, (unsigned)K, (unsigned)std::min<int64_t>(t.groups, 65535));
-#define WM_BC(VBv, VECv)                                                                                       \
-    launch_kernel((bwd_cols_kernel<OP, VBv, VECv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV, accV, \
-                  ws.as<float>(), O, R, C, t)
-    if (vb) { if (vec) WM_BC(true, true); else WM_BC(true, false); }
-    else { if (vec) WM_BC(false, true); else WM_BC(false, false); }
+#define WM_BC(VBv, VECv, FOLDv)                                                                                   \
+    launch_kernel((bwd_cols_kernel<OP, VBv, VECv, FOLDv>), grid, dim3(kBlock), 0, st, g, F, V, o, gF, accF, gV,   \
+                  accV, ws.as<float>(), O, R, C, t)
+    if (t.fold) {
+        if (vb) { if (vec) WM_BC(true, true, true); else WM_BC(true, false, true); }
+        else { if (vec) WM_BC(false, true, true); else WM_BC(false, false, true); }
+    } else {
+        if (vb) { if (vec) WM_BC(true, true, false); else WM_BC(true, false, false); }
+        else { if (vec) WM_BC(false, true, false); else WM_BC(false, false, false); }
+    }
 #undef WM_BC
     WM_TRY(check_launch("wm_binary_bwd(cols)"));
-    if (gV && K > 1) return launch_colsum_finalize(ws.as<float>(), gV, accV, K, C, O, st);
+    if (gV && K > 1) return launch_colsum_finalize(ws.as<float>(), gV, accV, K, nv, O, st);
     return WM_OK;
 }
 
@@ -905,12 +927,25 @@ int launch_binary_bwd(const float* g, const float* a, const float* b, const floa
             const int64_t O = nd == 3 ? size[0] : 1, R = size[nd - 2];
             // bwd_colsum_kernel keeps the wide aligned [R, C] it was shaped
             // for (one row per step, 1024-column tiles).
-            const ColTile t = vec ? col_tile(O, R, C / 4, col_rows<OP, true>())
-                                  : col_tile(O, R, C, col_rows<OP, false>());
+            const ColTile t = vec ? col_tile(O, R, C / 4, col_rows<OP, true>(), 0)
+                                  : col_tile(O, R, C, col_rows<OP, false>(), 0);
             if (!(O == 1 && vec && C >= kBlock * 4) && t.tiles <= kMaxGrid)
                 return launch_cols<OP>(t, vb, vec, g, F, V, o, gF, accF, gV, accV, O, R, C);
         } else if (nd == 3 && sv[0] == 0 && sv[1] == 1 && sv[2] == 0) {
-            return launch_channel<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, size[0], size[1], C);
+            const int64_t O = size[0], K = size[1], U = vec ? C / 4 : C;  // U: units per plane
+            // Many channels of short planes share workgroups.  Add, with the
+            // one-thread-per-channel kernel before, a workgroup per channel and
+            // so: [2, 65536, 4] 12.7, 50.4 and 5.7 us, [4, 500000, 3] 63, 416
+            // and 17, [16, 4096, 16] 115, 6.5 and 5.6.  Few channels fill their
+            // workgroups better alone ([32, 2048, 49] 12.0 against 14.1), and
+            // so do long planes (pow over [2, 65536, 196] 188 against 209).
+            if (K >= 4096 && U <= 32) {
+                const ColTile t = vec ? col_tile(1, O, K * U, col_rows<OP, true>(), (int)U)
+                                      : col_tile(1, O, K * U, col_rows<OP, false>(), (int)U);
+                if (t.tiles <= kMaxGrid)
+                    return launch_cols<OP>(t, vb, vec, g, F, V, o, gF, accF, gV, accV, 1, O, K * C);
+            }
+            if (K <= kMaxGrid) return launch_channel<OP>(vb, vec, g, F, V, o, gF, accF, gV, accV, O, K, C);
         }
     }
 
