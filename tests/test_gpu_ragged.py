@@ -351,3 +351,16 @@ def backward_pace(wm, full, vec):
                                       ((4, 200000, 3), (1, 200000, 1))])
 def test_broadcast_backward_pace(wm, full, vec):
     assert backward_pace(wm, full, vec) < 5.0
+
+
+def test_layernorm_backward_pace(wm):
+    """Wide rows over few enough workgroups that their partials are a small part
+    of the traffic (1.13 times a copy; eight workgroups per CU: 1.40)."""
+    rows, n = 16384, 2048
+    g, x, gx = (wm.DeviceArray((rows, n)) for _ in range(3))
+    gamma, dg, db = (wm.DeviceArray((n,)) for _ in range(3))
+    mean, inv = wm.DeviceArray((rows,)), wm.DeviceArray((rows,))
+    for d in (g, x, gamma, mean, inv):
+        d.fill(1.0)
+    assert pace(wm, 12 * rows * n, lambda: wm.call("wm_layernorm_bwd", g.vp, x.vp, gamma.vp, mean.vp, inv.vp, rows, n,
+                                                   gx.vp, 0, dg.vp, 0, db.vp, 0)) < 1.27

@@ -1123,9 +1123,15 @@ int launch_ln_bwd(const float* g, const float* x, const float* gamma, const floa
     // flight): [8192, 768] 17.3 + 4.5 us for the two dispatches, against 16.7 + 6.2
     // at two per CU and 17.2 + 9.8 at four; [32768, 128] 12.9 + 4.4 at four
     // against 27.9 + 4.5 at one.  Wider rows: at least 8 rows per workgroup, or 4
-    // when there are few (of 32 before: [768, 8192] 82 -> 23 us).
+    // when there are few (32 rows each: [768, 8192] 83 us against 28), on at most
+    // two workgroups per CU, one for rows of two float4s per thread of 1024 (more
+    // leave more partials to write and read than they hide: [16384, 2048] 89.5
+    // us at 8 per CU, 71.4 at two; [8192, 4096] 84.1 at four, 76.9; [8192, 8192]
+    // 169 at four, 152 at two, 145 at one).
     const bool wave = tc.nt == 64;
-    const int per_cu = !wave ? ln_waves(tc.nt) * 2 : want_p && tc.items > 1 ? 1 : 4;
+    const int per_cu = !want_p ? (wave ? 4 : ln_waves(tc.nt) * 2)
+                       : wave  ? (tc.items > 1 ? 1 : 4)
+                               : (tc.nt == 1024 && tc.items > 1 ? 1 : 2);
     int64_t G = std::min<int64_t>(wave ? (rows + 3) / 4 : rows, (int64_t)num_cus() * per_cu);
     const int64_t least = wave || rows >= 1024 ? 8 : 4;
     if (want_p) G = std::max<int64_t>(1, std::min<int64_t>(G, (rows + least - 1) / least));
