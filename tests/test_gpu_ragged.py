@@ -236,6 +236,14 @@ def test_strided_reductions_short_axis(wm, outer, n, inner):
             assert i is None or np.array_equal(i, ri), op
 
 
+# The lines between sixteen waves on the whole axis and chunks of it: 160 and 256
+# positions of few float4 tiles, 512 of 192 tiles (3/4 of the CUs), of 256 float tiles.
+@pytest.mark.parametrize("outer,n,inner", [(1, 160, 64), (1, 161, 64), (2, 256, 256), (2, 257, 256), (191, 300, 4),
+                                           (192, 300, 4), (192, 513, 4), (256, 512, 3), (257, 512, 3)])
+def test_strided_reductions_route_lines(wm, outer, n, inner):
+    test_strided_reductions_short_axis(wm, outer, n, inner)
+
+
 # Broadcast forwards over rows of whole float4s that are not whole tiles, the
 # broadcast operand along the row, along the outer dims and both.
 @pytest.mark.parametrize("op", ["add", "div", "max"])

@@ -967,13 +967,20 @@ int launch_cols(const float* x, int64_t outer, int64_t n, int64_t inner, float* 
     if (outer * tiles < target_blocks)
         K = std::min<int64_t>((target_blocks + outer * tiles - 1) / (outer * tiles), (n + 127) / 128);
     K = std::max<int64_t>(std::min<int64_t>(K, 4096), 1);
-    // Where that asks for chunks of a short n, 16 waves on the whole of it (at
-    // most 20 positions each, 32 where half the CUs have a workgroup) spare the
-    // second dispatch.  Mean / max, both passes before and one now:
-    // [64, 197, 768] 15.8 / 15.7 -> 11.0 / 11.0 us, [197, 402, 3] 7.5 / 8.2 -> 5.4 /
-    // 6.0, [1, 300, 10] 5.1 / 6.1 -> 4.2 / 5.0; but [16, 512, 64] 7.8 / 8.2 against 8.5 /
-    // 11.4 and [1, 1000, 768] 8.9 / 9.2 against 20.8 / 22.0, which keep their chunks.
-    const bool tall = K > 1 && n <= (2 * outer * tiles >= num_cus() ? 512 : 320);
+    // Where that asks for chunks of a short n, 16 waves on the whole of it may
+    // spare the second dispatch.  Chunks / 16 waves, us, in float4s: with 3/4 of
+    // the CUs or more busy up to n = 512 ([64, 197, 768] mean 10.1 / 8.7, max 12.2 /
+    // 10.8, [16, 512, 4096] 25.2 / 20.2 and 27.5 / 22.6); with fewer, the sums up to
+    // 256 and the max family up to 160 ([32, 256, 256] 7.7 / 6.3 and [32, 160, 256]
+    // 7.9 / 7.9; but [32, 300, 256] 7.9 / 9.0, and max [32, 200, 256] 8.1 / 9.4, [8,
+    // 300, 4096] 11.4 / 12.2).  In floats: up to n = 512 on at most a workgroup per CU
+    // ([197, 402, 3] max 10.3 / 8.1; but [128, 200, 257], 640 workgroups, 12.4 / 15.3).
+    const int64_t wgs = outer * tiles;
+    const int64_t most = !vec                      ? (wgs <= num_cus() ? 512 : 0)
+                         : 4 * wgs >= 3 * num_cus() ? 512
+                         : KIND == 0                ? 256
+                                                    : 160;
+    const bool tall = K > 1 && n <= most;
     if (tall) K = 1;
     const int64_t chunk = (n + K - 1) / K;
     K = std::max<int64_t>(1, (n + chunk - 1) / chunk);
