@@ -372,3 +372,26 @@ def test_layernorm_backward_pace(wm):
         d.fill(1.0)
     assert pace(wm, 12 * rows * n, lambda: wm.call("wm_layernorm_bwd", g.vp, x.vp, gamma.vp, mean.vp, inv.vp, rows, n,
                                                    gx.vp, 0, dg.vp, 0, db.vp, 0)) < 1.27
+
+
+@pytest.mark.parametrize("offset", [0, 3])
+@pytest.mark.parametrize("rows,cols", [(3, 5), (3, 6), (70, 17), (130, 20), (130, 21), (9, 159), (9, 161), (7, 319),
+                                       (7, 321), (5, 1020), (5, 1021), (3, 1499), (3, 1502), (3, 1503), (3, 1507)])
+def test_cross_entropy_rows_a_little_longer_than_their_lanes(wm, rows, cols, offset):
+    """Rows whose lanes or tile take a second float4, at the ends of each."""
+    test_cross_entropy_rows_at_any_alignment(wm, rows, cols, offset)
+
+
+def test_cross_entropy_backward_pace(wm):
+    """Rows of one float4 more than a workgroup's lanes at some shifts: 1.5 times a
+    copy (2.5 with a tile of its own for it)."""
+    rows, cols = 32768, 1023
+    x, gx = wm.DeviceArray((rows, cols)), wm.DeviceArray((rows, cols))
+    lab, g = wm.DeviceArray((rows,)), wm.DeviceArray((1,))
+    stats, loss = wm.DeviceArray((rows, wm.CE_STATS)), wm.DeviceArray((1,))
+    for d in (x, lab, g):
+        d.fill(1.0)
+    wm.call("wm_cross_entropy_fwd", x.vp, lab.vp, rows, cols, stats.vp, loss.vp)
+    p = pace(wm, 8 * rows * cols, lambda: wm.call("wm_cross_entropy_bwd", x.vp, lab.vp, stats.vp, g.vp, gx.vp, 0, rows,
+                                                  cols))
+    assert p < 1.95

@@ -268,11 +268,14 @@ __global__ void __launch_bounds__(256) head_bwd_tile_kernel(const float* __restr
 // Rows of any length: the same tiles, shifted per row so that the gradient's
 // stores start on a 128-byte line (16 bytes for short rows; the loads then do
 // too, or are 128 bits at 4-byte alignment); the float4s that cross either end
-// of a row go element by element.  Rows of fewer than 256 float4s share a
-// workgroup, 2^lpr_log2 lanes each.  [2048, 50257] cross entropy: 248 -> 147
-// us against a workgroup per row with one float per thread (172 with unshifted
-// tiles, 152 shifted to 16 bytes only); 16384 rows of 13 classes 8.6 -> 4.2 us.
-template <int MODE>
+// of a row are loaded and stored element by element, their four loads out before
+// the first is used.  Short rows share a workgroup, 2^lpr_log2 lanes each.
+// [2048, 50257] cross entropy: 137 us, 248 with a workgroup per row and one
+// float per thread (172 with unshifted tiles, 152 shifted to 16 bytes only, 146
+// with the end elements one after the other); 131072 rows of 17 classes 14.5
+// us against 50.3, 65536 of 127 22.6 against 31.9.
+// MORE: one tile, some of whose lanes may take a second float4.
+template <int MODE, bool MORE>
 __global__ void __launch_bounds__(256) head_bwd_ragged_kernel(const float* __restrict__ x,
                                                                const float* __restrict__ labels,
                                                                const float* __restrict__ stats,
@@ -288,32 +291,45 @@ __global__ void __launch_bounds__(256) head_bwd_ragged_kernel(const float* __res
         const int64_t r = r0 + sub;
         if (r >= rows) continue;
         const int lead = (int)((((uintptr_t)gx >> 2) + (uintptr_t)(r * cols)) & lead_mask);
-        const int64_t c0 = ((int64_t)blockIdx.x * 256 + lane) * 4 - lead;
+        int64_t c0 = ((int64_t)blockIdx.x * 256 + lane) * 4 - lead;
         if (c0 >= cols) continue;
         const HeadRow h = head_row<MODE>(stats, labels[r], r, cols, scale);
         const float* xr = x + r * cols;
         float* gr = gx + r * cols;
-        if (c0 >= 0 && c0 + 3 < cols) {
-            const float4 xv = MODE != kOneHot ? ld_unaligned(xr + c0) : make_float4(0.f, 0.f, 0.f, 0.f);
-            const float4 ov = acc ? ld_stream(gr + c0) : make_float4(0.f, 0.f, 0.f, 0.f);
-            float d0 = head_elem<MODE>(xv.x, c0 == h.lab, h, scale, alpha);
-            float d1 = head_elem<MODE>(xv.y, c0 + 1 == h.lab, h, scale, alpha);
-            float d2 = head_elem<MODE>(xv.z, c0 + 2 == h.lab, h, scale, alpha);
-            float d3 = head_elem<MODE>(xv.w, c0 + 3 == h.lab, h, scale, alpha);
-            if (acc) {
-                d0 = ov.x + d0; d1 = ov.y + d1; d2 = ov.z + d2; d3 = ov.w + d3;
+        do {
+            const bool whole = c0 >= 0 && c0 + 3 < cols;
+            float v[4] = {0.f, 0.f, 0.f, 0.f}, old[4] = {0.f, 0.f, 0.f, 0.f}, d[4];
+            if (whole) {
+                if (MODE != kOneHot) {
+                    const float4 q = ld_unaligned(xr + c0);
+                    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+                }
+                if (acc) {
+                    const float4 q = ld_stream(gr + c0);
+                    old[0] = q.x; old[1] = q.y; old[2] = q.z; old[3] = q.w;
+                }
+            } else {  // past an end: the row's first or last element, not stored
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int64_t c = c0 + e < 0 ? 0 : c0 + e < cols ? c0 + e : cols - 1;
+                    if (MODE != kOneHot) v[e] = ld_stream1(xr + c);
+                    if (acc) old[e] = ld_stream1(gr + c);
+                }
             }
-            st_stream(gr + c0, make_float4(d0, d1, d2, d3));
-        } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int64_t c = c0 + e;
-                if (c < 0 || c >= cols) continue;
-                float d = head_elem<MODE>(MODE != kOneHot ? ld_stream1(xr + c) : 0.f, c == h.lab, h, scale, alpha);
-                if (acc) d = ld_stream1(gr + c) + d;
-                st_stream1(gr + c, d);
+                d[e] = head_elem<MODE>(v[e], c0 + e == h.lab, h, scale, alpha);
+                if (acc) d[e] = old[e] + d[e];
             }
-        }
+            if (whole) {
+                st_stream(gr + c0, make_float4(d[0], d[1], d[2], d[3]));
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (c0 + e >= 0 && c0 + e < cols) st_stream1(gr + c0 + e, d[e]);
+            }
+            c0 += 4 << lpr_log2;
+        } while (MORE && c0 < cols);
     }
 }
 
@@ -571,16 +587,24 @@ int launch_head_bwd(const float* x, const float* labels, const float* stats, con
         launch_kernel((head_bwd_tile_kernel<MODE>), dim3(grid_for(rows * tiles, 1, 1 << 12)), dim3(256), 0,
                       stream(), x, labels, stats, loss_grad, gx, acc, rows, cols, alpha);
     } else {
-        // Long rows shift to whole 128-byte lines, short ones to 16 bytes; n4:
-        // float4s of a row at any shift.
+        // Long rows shift to whole 128-byte lines, short ones to 16 bytes.  As
+        // many lanes as a row has float4s or a quarter fewer, and one tile up to
+        // 384 float4s at any shift: the few lanes that take a second float4 cost
+        // less than the idle ones of twice the lanes or of another tile ([8192,
+        // 1023] 17.7 us against 27.4, [65536, 129] 23.8 against 36.8).
         const unsigned mask = cols >= 1024 ? 31u : 3u;
         const int64_t n4 = (cols + mask + 3) / 4;
         int lg = 0;
-        while (lg < 8 && (1 << lg) < n4) ++lg;
+        while (lg < 8 && (1 << lg) + (1 << lg) / 4 < (cols + 3) / 4) ++lg;
         const int64_t groups = (rows + (256 >> lg) - 1) / (256 >> lg);
-        const dim3 grid((unsigned)((n4 + 255) / 256), (unsigned)std::min<int64_t>(groups, 65535));
-        launch_kernel((head_bwd_ragged_kernel<MODE>), grid, dim3(256), 0, stream(), x, labels, stats, loss_grad, gx,
-                      acc, rows, cols, alpha, lg, mask);
+        const bool more = n4 <= 384;
+        const dim3 grid(more ? 1u : (unsigned)((n4 + 255) / 256), (unsigned)std::min<int64_t>(groups, 65535));
+        if (more)
+            launch_kernel((head_bwd_ragged_kernel<MODE, true>), grid, dim3(256), 0, stream(), x, labels, stats,
+                          loss_grad, gx, acc, rows, cols, alpha, lg, mask);
+        else
+            launch_kernel((head_bwd_ragged_kernel<MODE, false>), grid, dim3(256), 0, stream(), x, labels, stats,
+                          loss_grad, gx, acc, rows, cols, alpha, lg, mask);
     }
     return check_launch(what);
 }
