@@ -190,12 +190,14 @@ __global__ void __launch_bounds__(kBlock) bwd_colsum_kernel(const float* __restr
 // Few columns over many partial rows (a Linear bias gradient, 1024 columns
 // over 1024 row groups) take 4 columns per workgroup, so that the grid has
 // ~256 workgroups (64 columns left 16 workgroups each walking 256 rows per
-// wave: 13.6 us); from 2048 columns on, 64 columns with 16 groups read whole
+// wave: 13.6 us).  From 1280 columns on, 64 columns with 16 groups read whole
 // lines with as many rows in flight ([512, 4096] partials 5.2 us against 11.5
-// for 16 columns with 16 groups); at most 8 partial rows of 65536 columns or
-// more, a thread per column (a row vector's gradient over [2, 500000] 9.8 us
-// with 64 columns and their tree, 7.4 so; [4, 2^20] 19.3 and 14.2; with 32
-// partial rows the tree is 1 us faster).
+// for 16 columns with 16 groups; bias gradients over [1000, 1280] 10.1 against
+// 11.2 with 4 columns, [4096, 2000] 20.0 and 22.6; [65536, 1024] 106 and 104).
+// At most 8 partial rows of 65536 columns or more take a thread per column (a
+// row vector's gradient over [2, 500000] 9.8 us with 64 columns and their
+// tree, 7.4 so; [4, 2^20] 19.3 and 14.2; with 32 partial rows the tree is 1 us
+// faster).
 template <int S, int NT>
 __global__ void __launch_bounds__(NT) colsum_finalize_kernel(const float* __restrict__ part, float* __restrict__ out,
                                                                   int acc, int64_t K, int64_t C, int64_t O) {
@@ -230,7 +232,7 @@ int launch_colsum_finalize(const float* part, float* out, int acc, int64_t K, in
                   dim3(NT), 0, st, part, out, acc, K, C, O)
     if (cols >= 256 * want && K <= 8) WM_CF(256, kBlock);
     else if (cols >= 64 * want) WM_CF(64, kBlock);
-    else if (cols >= 8 * want) WM_CF(64, 1024);
+    else if (cols >= 5 * want) WM_CF(64, 1024);
     else WM_CF(4, kBlock);
 #undef WM_CF
     return check_launch("wm_binary_bwd(colsum finalize)");
