@@ -136,6 +136,16 @@ def test_fused_epilogue(wm, shape, accumulate, bounds):
     assert ok, f"g.grad off by {worst:.3g}x tolerance"
 
 
+# The backward's tiles: one, two and four waves side by side with and without a
+# part-filled last one, by single elements; float4 groups missing at a row's end,
+# which only inputs and gradients past 256 MB take.
+@pytest.mark.parametrize("shape,accumulate", [((70, 448), False), ((33, 640), True), ((50, 768), False),
+                                              ((41, 772), True), ((41, 900), False), ((9, 3000), True),
+                                              ((200, 65), False), ((345, 65100), False)])
+def test_fused_epilogue_backward_tiles(wm, shape, accumulate):
+    test_fused_epilogue(wm, shape, accumulate, (LO, HI))
+
+
 def test_fused_matches_composed_tensor_ops(wm):
     """The fused kernels equal the chain of drop-in Tensor ops on fp32 copies
     of the fp16 inputs (reshape to 2-D, mean(1, keepdim), backward)."""

@@ -382,14 +382,22 @@ int wm_epilogue_f16_bwd(const float* dm, const uint16_t* h, const uint16_t* res,
     if (!dm || !h || !res || !g) return set_error(WM_ERR_INVALID, "wm_epilogue_f16_bwd: null pointer");
     if (!gh && !gres && !gg) return WM_OK;
     WM_CHECK_INIT();
-    const bool vec = cols % 4 == 0 && cols >= 256 && aligned16(h) && aligned16(res) && aligned16(g) &&
+    // 128-bit accesses where whole waves of them cover a row, or where the
+    // inputs and gradients exceed the 256 MB of the last cache; rows that leave
+    // part of a wave's two groups empty stream faster by single elements while
+    // they fit ([16384, 1000] 43 us against 51, [8192, 768] 20.7 against 25.5; but
+    // [32768, 768] 103 against 66, [1000, 65540] 276 against 201).
+    const bool whole = cols % 512 == 0;
+    const bool vec = cols % 4 == 0 && cols >= 256 && (whole || rows * cols > ((int64_t)256 << 20) / 12) && aligned16(h) && aligned16(res) && aligned16(g) &&
                      (!gh || aligned16(gh)) && (!gres || aligned16(gres));
-    // A wave covers 512 columns (64 of a short or unaligned row); as many waves
-    // side by side along a row as divide it, a workgroup's other waves on the
-    // next rows.
+    // A wave covers 512 columns (64 by single elements); as many waves side by
+    // side along a row as leave at most an eighth of them without columns, a
+    // workgroup's other waves on the next rows.
     const int64_t wave_tiles = (cols + (vec ? 511 : 63)) / (vec ? 512 : 64);
-    const int wpr_log2 = wave_tiles % 4 == 0 ? 2 : wave_tiles % 2 == 0 ? 1 : 0;
-    const int64_t rpb = 4 >> wpr_log2, col_tiles = wave_tiles >> wpr_log2;
+    auto wgs = [&](int l) { return (wave_tiles + (1 << l) - 1) >> l; };
+    int wpr_log2 = 2;
+    while (wpr_log2 > 0 && 7 * (wgs(wpr_log2) << wpr_log2) > 8 * wave_tiles) --wpr_log2;
+    const int64_t rpb = 4 >> wpr_log2, col_tiles = wgs(wpr_log2);
     // ~4 workgroups per CU, each row group of at least 4 rows per wave: each
     // thread folds its columns' dg partials over its rows, and the second
     // pass reads K partials per column.  With 16 rows per thread at least and a
@@ -405,7 +413,7 @@ int wm_epilogue_f16_bwd(const float* dm, const uint16_t* h, const uint16_t* res,
 #define WM_EPI_BWD(V, F, A)                                                                                      \
     launch_kernel((epilogue_bwd_kernel<V, F, A>), grid, dim3(kBlock), 0, stream(), dm, h, res, g, gh, acc_h, gres, \
                   acc_res, ws.as<float>(), rows, cols, lo, hi, wpr_log2)
-    if (vec && cols % 512 == 0) { if (fc) WM_EPI_BWD(true, true, true); else WM_EPI_BWD(true, false, true); }
+    if (vec && whole) { if (fc) WM_EPI_BWD(true, true, true); else WM_EPI_BWD(true, false, true); }
     else if (vec) { if (fc) WM_EPI_BWD(true, true, false); else WM_EPI_BWD(true, false, false); }
     else { if (fc) WM_EPI_BWD(false, true, false); else WM_EPI_BWD(false, false, false); }
 #undef WM_EPI_BWD
