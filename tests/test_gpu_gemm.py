@@ -9,6 +9,8 @@ exact in fp32 (small integers).  Sizes past the oracle's seconds are checked
 against numpy's float64 product, which test_oracle_gemm.py pins to the fp64
 oracle.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -149,11 +151,27 @@ def test_gemm_k_zero_and_empty(wm):
 @pytest.mark.parametrize("mnk", [(128, 128, 1), (130, 140, 100), (200, 129, 256), (128, 256, 257)], ids=str)
 def test_gemm_one_level_batch_padded_alpha_accumulate(wm, mnk):
     """One-level batches of untransposed products with padded rows and
-    problem strides, alpha and accumulation (the shapes up to k = 256 with
-    m, n >= 128 take rocBLAS's strided-batched route by default, k = 257
-    this library's kernel); the padding of C stays untouched."""
-    m, n, k = mnk
-    P, pad, gap = 3, 3, 11
+    problem strides, alpha and accumulation (three problems: the small-tile
+    kernel by default, the 128-row ones with the library route off); the
+    padding of C stays untouched."""
+    check_batch_padded(3, *mnk)
+
+
+@pytest.mark.parametrize("case", [(70, 200, 129, 96), (10, 209, 392, 256), (27, 280, 128, 255), (90, 128, 130, 12)],
+                         ids=str)
+def test_gemm_library_strided_batches(wm, route, case):
+    """Batches of untransposed products with m, n >= 128, k <= 256 that are not
+    all-interior go to rocBLAS's strided-batched call by default (no kernel of this
+    library runs), also where their 128-row tiles are fewer than the CUs."""
+    before, after = C.c_int64(), C.c_int64()
+    wm.call("wm_launch_count", C.byref(before))
+    check_batch_padded(*case)
+    wm.call("wm_launch_count", C.byref(after))
+    assert (after.value == before.value) == (route == 1)
+
+
+def check_batch_padded(P, m, n, k):
+    pad, gap = 3, 11
     lda, ldb, ldc = k + pad, n + pad, n + pad
     sa, sb, sc = m * lda + gap, k * ldb + gap, m * ldc + gap
     A, B = rng_normal((P, m, k), 45), rng_normal((P, k, n), 46)
@@ -179,7 +197,9 @@ def test_gemm_one_level_batch_padded_alpha_accumulate(wm, mnk):
                                   (17, 1024, 1024, 64, True), (16, 1024, 512, 128, False)], ids=str)
 def test_gemm_dma_batches(wm, case):
     """One-level batches whose tiles are all interior (m, n multiples of 128,
-    k of 64, 16-byte rows) run on the direct-to-LDS kernel (untransposed here):
+    k of 64, 16-byte rows) run on the direct-to-LDS kernel (untransposed here;
+    the ones of few tiles only with the library route off, the small-tile kernel
+    takes them by default):
     k = 64 and 192 (one and three rounds of its four stage buffers), 1024;
     17 problems of 64 tiles take two problems per workgroup with a last
     workgroup of one; padded rows (pad 4 keeps the rows 16-byte aligned) and
@@ -216,8 +236,8 @@ def test_gemm_dma_batches(wm, case):
 @pytest.mark.parametrize("case", [(3, 128, 256, 64), (2, 256, 128, 192), (4, 256, 256, 384), (3, 1024, 128, 1024),
                                   (17, 1024, 1024, 64)], ids=str)
 def test_gemm_dma_transposed(wm, trans, case):
-    """The direct-to-LDS kernels with transposed operands (A stored k x m,
-    B stored n x k): the k-contiguous and row-contiguous stagings swap sides;
+    """The direct-to-LDS kernels (by default the small-tile kernel where the
+    tiles are few) with transposed operands (A stored k x m, B stored n x k): the k-contiguous and row-contiguous stagings swap sides;
     k <= 256 on the three-buffer kernel, k = 384 on the four-buffer one.
     Padded leading dimensions and gaps between problems, alpha, accumulation
     and a bias; 17 problems of 64 tiles take two problems per workgroup."""
@@ -256,8 +276,8 @@ def test_gemm_dma_transposed(wm, trans, case):
 @pytest.mark.parametrize("shape", [(4, 1024, 128, 1024), (64, 256, 128, 256), (8, 512, 128, 512)], ids=str)
 def test_bmm_backward_on_dma_kernel(wm, shape):
     """bmm's closure at attention-like shapes: its two products (g b^T and
-    a^T g) run on the direct-to-LDS kernel; both gradients, overwritten and
-    accumulated."""
+    a^T g) run on the direct-to-LDS kernel (the smaller ones by default on the
+    small-tile kernel); both gradients, overwritten and accumulated."""
     P, t, hd, t2 = shape
     a, b = rng_normal((P, t, hd), 94), rng_normal((P, hd, t2), 95)
     g = rng_normal((P, t, t2), 96)
@@ -306,7 +326,7 @@ def test_gemm_two_level_per_head_interior(wm, kind, hd):
 @pytest.mark.parametrize("case", [(129, 1024, 32), (5, 256, 96), (3, 384, 1024)], ids=str)
 def test_gemm_dma32_transposed_a(wm, case):
     """op(A) = A^T with n = 64 (the attention backward's dV and dK) on the
-    32-k direct-to-LDS kernel: one stage (k = 32), three stages rotating over
+    32-k direct-to-LDS kernel (few tiles by default on the small-tile one): one stage (k = 32), three stages rotating over
     the three buffers (k = 96), k = 1024; 129 problems of 8 tiles take two
     problems per workgroup with a last one of one; padded rows, gaps between
     problems, alpha, accumulation and a bias."""

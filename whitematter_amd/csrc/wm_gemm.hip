@@ -1420,37 +1420,54 @@ int launch_dma32(GemmParams P, int64_t tiles) {
 
 // Which kernel takes a product that the library does not: an estimate of each
 // form's time, in us, from how a grid of such tiles ran on MI355X (m, n, k
-// from 1 to 8192, all transposes): a start, then the longer of one wave's
-// chain of k steps and the chip's rate over all tiles.
-//   16 x 16, k over 4 or 16 waves   2.8 + max(0.50 S, T (WK 0.00055 + steps 0.00038))
-//   32 x 32, k over 4 waves         3.3 + max(0.45 S, T (0.0022 + steps 0.00056))
-//   64 x 64, a wave per quarter     4.0 + max(0.41 S, T (0.0022 + steps 0.0018))
-//   128-row tiles                   5.0 + max(2.5 nk (1.5 from LDS), T nk 0.0105), 5 more when k is split
-// (S: k steps of one wave, T: tiles of all problems, nk: 32-k stages; half
-// the rate's term for 64-wide tiles.)  Measured on both sides, small / 128-row:
+// from 1 to 8192, up to 400 problems, all transposes): a start, then the longer
+// of one wave's chain of k steps and the chip's rate over all tiles.
+//   16 x 16, k over 4 or 16 waves   2.8 + max(0.50 S c, T (WK 0.00055 + steps 0.00038))
+//   32 x 32, k over 4 waves         3.3 + max(0.45 S c, T (0.0022 + steps 0.00056))
+//   64 x 64, a wave per quarter     4.0 + max(0.41 S c, T' (0.0022 + steps 0.0018))
+//   128-row tiles                   5.0 + max(6 + 2.5 nk, T" (0.01 + 0.0095 nk)), 5 more when k is split
+// S: k steps of one wave; T: tiles of all problems (and k slices), T' in whole
+// rounds of the CUs, T" half way between (a tile's time on a CU shrinks when it
+// is alone there); nk: 32-k stages, 1.5 nk and no 6 for the direct-to-LDS
+// kernels, 0.0135 at unaligned rows, half T" and 3.6 for 64-wide tiles.  c: 1, but from k = 1024 on 1.2, and 2.5 over 48 tiles or
+// more, where neither or both operands are transposed (one is read along k and
+// the other across it).
+// A batch that the library takes starts at 7.5 us there; small tiles take it if
+// they end by 6.5.  Over 7285 such products drawn at random, small tiles were
+// chosen where the 128-row kernels or the library are more than 5 % faster 28
+// times, by up to 1.35x (190 times, up to 2.8x, when a batch below a tile per
+// CU went by the estimates alone).  Measured on both sides, small / 128-row:
 //   (64, 128, 784) 5.5 / 83, (784, 128, 64)^T 3.5 / 12.8, (16, 512, 512) 5.2 / 50,
 //   (4096, 10, 768) 6.7 / 62, (32, 32, 8192) 20 / 30, (5912, 1392, 30) 18 / 34,
-//   (3072, 768, 128) 16.3 / 15.5, (2624, 2576, 221) 51 / 60 us.
+//   (3072, 768, 128) 16.3 / 15.5, (2624, 2576, 221) 51 / 60 us; small / library:
+//   27 of (280, 128, 256) 24.0 / 8.6, 26 of (320, 256, 256) 31 / 16.7, 6 of (139,
+//   374, 18) 5.1 / 7.6.
 enum SmallForm { kNoSmall, kSmall16x4, kSmall16x16, kSmall32x4, kSmall64 };
 
 double big_us(const GemmParams& P, bool lds_dma, bool narrow, bool vec, int64_t work) {
     const int64_t ks = lds_dma ? 1 : choose_kslices(work, P.k);
     const double nk = std::ceil((double)P.k / (double)ks / kBK);
-    const double stage = (vec ? 0.0105 : 0.016) * (narrow ? 0.5 : 1.0);
-    return 5.0 + std::max((lds_dma ? 1.5 : 2.5) * nk, (double)work * ks * nk * stage) + (ks > 1 ? 5.0 : 0.0);
+    const double half = narrow ? 0.5 : 1.0;
+    const double chain = lds_dma ? 1.5 * nk : 2.5 * nk + (narrow ? 3.6 : 6.0);
+    const double all = (double)work * ks, cus = (double)num_cus();
+    const double rate = 0.5 * (all + std::ceil(all / cus) * cus) * (nk * (vec ? 0.0095 : 0.0135) + 0.01) * half;
+    return 5.0 + std::max(chain, rate) + (ks > 1 ? 5.0 : 0.0);
 }
 
-SmallForm choose_small(const GemmParams& P, double limit_us) {
+SmallForm choose_small(bool ta, bool tb, const GemmParams& P, double limit_us) {
     // 32-bit lane offsets: at most 32 rows of the leading dimension in bytes.
     if (P.lda > (1 << 23) || P.ldb > (1 << 23) || P.k > INT_MAX) return kNoSmall;
     auto tiles = [&](int64_t b) { return (double)((P.m + b - 1) / b) * (double)((P.n + b - 1) / b); };
-    if (tiles(16) > (double)INT_MAX) return kNoSmall;
     SmallForm best = kNoSmall;
     auto consider = [&](SmallForm f, int64_t blk, double start, double per_step, double per_tile, double rate,
                         int64_t kstep, int64_t wk) {
-        const double steps = std::ceil((double)P.k / (double)kstep);
-        const double us = start + std::max(per_step * std::ceil(steps / (double)wk),
-                                           tiles(blk) * (double)P.batch * (per_tile + steps * rate));
+        // The grid's x has fewer than 2^32 threads (1024 at most per tile).
+        if (tiles(blk) >= (double)(1 << 22)) return;
+        const double steps = std::ceil((double)P.k / (double)kstep), all = tiles(blk) * (double)P.batch;
+        const double c = ta == tb && P.k >= 1024 ? (all >= 48 ? 2.5 : 1.2) : 1.0;
+        const double cus = (double)num_cus(), rounds = f == kSmall64 ? std::ceil(all / cus) * cus : all;
+        const double us = start + std::max(per_step * c * std::ceil(steps / (double)wk),
+                                           rounds * (per_tile + steps * rate));
         if (us < limit_us) {
             limit_us = us;
             best = f;
@@ -1517,19 +1534,19 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
     hipStream_t s = stream();
     P.kslices = 1;
     P.group = 1;
-    // The library keeps its plain large products, and its batched ones that
-    // fill the chip; the estimates above choose between small tiles, the
-    // direct-to-LDS kernels where a batch fits them, and gemm_kernel for the
-    // rest.  With the library route off every product runs on the 128-row
-    // kernels.
+    // The library keeps the products it takes, but for batches of a few small
+    // tiles; the estimates above choose between small tiles, the direct-to-LDS
+    // kernels where a batch fits them, and gemm_kernel for the rest.  With the
+    // library route off every product runs on the 128-row kernels.
     const bool routed = g_library.load(std::memory_order_relaxed) != 0;
     const int64_t work = tm * tn * P.batch;
     // Unbatched products of more than dma3's k take launch_gemm's split, below.
     const bool dma = dma_fits(vec, P, tm * tn) && (P.batch > 1 || (!routed && P.k <= 256));
     const bool dma32 = narrow && dma32_fits(ta, tb, vec, P, tm * tn) && (P.batch > 1 || !routed);
-    const bool lib_first = library_takes(ta, tb, P) && (P.batch == 1 || work >= num_cus());
-    if (routed && P.k > 0 && !lib_first) {
-        const SmallForm f = choose_small(P, big_us(P, dma || dma32, narrow, vec, work));
+    const bool lib = library_takes(ta, tb, P);
+    if (routed && P.k > 0 && (!lib || P.batch > 1)) {
+        const double limit = lib && !dma ? 6.5 : big_us(P, dma || dma32, narrow, vec, work);
+        const SmallForm f = choose_small(ta, tb, P, limit);
         if (f != kNoSmall) return launch_small(f, ta, tb, P);
     }
     if (dma) {
@@ -1544,8 +1561,8 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
                            (!routed || split_beats_library(ta, tb, P, tm * tn));
     const DmaSplit split = dma_split ? choose_dma_split(P, tm * tn) : DmaSplit{1, 0};
     if (!dma_split) {
-        const int lib = try_library(ta, tb, P);
-        if (lib != 1) return lib;
+        const int r = try_library(ta, tb, P);
+        if (r != 1) return r;
     }
 
     // Split k: the partial products go to a workspace [batch][kslices][m][n]
@@ -1569,8 +1586,8 @@ int launch_gemm(bool ta, bool tb, const GemmParams& P0) {
         part.p = ws_alloc((size_t)(P.batch * kslices * mn) * sizeof(float));
         if (!part.p) {
             // The library needs none.
-            const int lib = dma_split ? try_library(ta, tb, F) : 1;
-            return lib != 1 ? lib : set_error(WM_ERR_NOMEM, "wm_gemm: split-k workspace");
+            const int r = dma_split ? try_library(ta, tb, F) : 1;
+            return r != 1 ? r : set_error(WM_ERR_NOMEM, "wm_gemm: split-k workspace");
         }
         P.c = part.as<float>();
         P.ldc = P.n;
