@@ -63,14 +63,14 @@ int wm_gemm(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alp
  * 128, k not of 64, rows not 16-byte aligned): 1 (default) = rocBLAS's
  * tuned fp32 kernels (sgemm / sgemm_strided_batched, atomics off), which
  * are faster there; 0 = this library's 128-row MFMA kernels for every
- * product.  On route 1 the products that leave most of the chip idle in 128-row
- * tiles (few rows or columns, small batches) run on this library's small-tile
- * kernel, and weight gradients A^T B over 4096 rows or more on the k split of
- * its interior-tile kernel where that fits and is faster.  mode 0 or 1 sets it, any other value only queries; returns the
- * route now in force.  The results agree with the reference within the same
- * fp32 summation error either way (both deterministic run to run).  No
- * counterpart in the reference (a routing switch, for tests and
- * measurements of each kernel).                                              */
+ * product.  On route 1 the products that leave most of the chip idle in
+ * 128-row tiles (few rows or columns, small batches) run on this library's
+ * small-tile kernel, and weight gradients A^T B over 3072 rows or more on the
+ * k split of its interior-tile kernel where that fits and is faster.  mode 0
+ * or 1 sets it, any other value only queries; returns the route now in force.
+ * The results agree with the reference within the same fp32 summation error
+ * either way (both deterministic run to run).  No counterpart in the
+ * reference (a routing switch, for tests and measurements of each kernel).   */
 int wm_gemm_library(int mode);
 
 /* Tensor::matmul, core/tensor.cpp:783-795: c[m, n] = a[m, k] @ b[k, n]. */

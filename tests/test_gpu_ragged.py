@@ -96,9 +96,9 @@ def test_small_products(wm, m, n, k, batch, ta, tb):
         assert np.array_equal(got[..., n:], c0[..., n:])  # past the rows: untouched
 
 
-# Weight gradients x^T dY on the k split of the direct-to-LDS kernel: the lines of
-# its rule (18 and 200 tiles, k = 4096), equal slices and a shorter last one, and
-# sizes next to the lines that the library keeps.
+# Weight gradients x^T dY on the k split of the direct-to-LDS kernel (with the library
+# route off; by default the library keeps some): 18 and 200 tiles, equal slices and
+# a shorter last one, and sizes that neither takes whole.
 @pytest.mark.parametrize("m,n,k", [(384, 768, 4096), (768, 384, 4160), (640, 512, 6848), (2560, 1280, 4096),
                                    (384, 768, 4032), (128, 2176, 4096), (1024, 1024, 4096), (384, 768, 4100)])
 @pytest.mark.parametrize("route", [0, 1])
@@ -124,6 +124,26 @@ def test_long_weight_gradients(wm, m, n, k, route):
             assert np.array_equal(got[0][:, n:], c0[:, n:])
     finally:
         wm.lib().wm_gemm_library(old)
+
+
+# Both sides of each line between the k split and the library (which launches no
+# kernel of this library).
+@pytest.mark.parametrize("m,n,k,split", [
+    (768, 384, 3072, True), (768, 384, 3008, False), (384, 768, 3072, False), (2176, 128, 3072, False),
+    (384, 1408, 3072, True), (256, 2048, 3072, False), (512, 1536, 3072, True), (896, 896, 3072, True),
+    (896, 1024, 3072, False), (1024, 1024, 3072, False), (640, 1664, 3072, True), (640, 2048, 3072, True),
+    (768, 1792, 3072, False), (640, 3328, 3072, True), (1024, 2176, 3072, False), (2432, 1280, 3072, True),
+    (3072, 1024, 3072, False), (1664, 1920, 3072, False), (2560, 1280, 3072, False)])
+def test_weight_gradient_route_lines(wm, m, n, k, split):
+    """Whole numbers: exact in float32 in any order."""
+    r = np.random.default_rng(seed_of("route", m, n, k))
+    x, dy = (r.integers(-3, 4, (k, w)).astype(np.float32) for w in (m, n))
+    before, after = C.c_int64(), C.c_int64()
+    wm.call("wm_launch_count", C.byref(before))
+    got = gemm(1, 0, m, n, k, 1.0, x.ravel(), m, dy.ravel(), n, np.zeros(m * n, np.float32), n, 0, None, 1, 1, None)
+    wm.call("wm_launch_count", C.byref(after))
+    assert (after.value > before.value) == split
+    assert np.array_equal(got.reshape(m, n), (x.T.astype(np.float64) @ dy).astype(np.float32))
 
 
 @pytest.mark.parametrize("offset", [0, 1, 2])

@@ -1207,10 +1207,12 @@ int64_t choose_kslices(int64_t work, int64_t k) {
 // contexts 45.7 / 64: two-level batches the library can only take as one
 // call per outer batch).  Batched products that gemm_dma_kernel takes run
 // there first (launch_gemm).  Unbatched products with m, n >= 128 and
-// k >= 256 (except the long-k weight gradients of split_beats_library), and the other one-level batches of untransposed products with
-// m, n >= 128, k <= 256, no bias and disjoint outputs, go to rocBLAS
-// (atomics off: the same bits on every run); the rest to gemm_kernel, and
-// while the library route is switched off (wm_gemm_library) every product
+// k >= 256 (except the long-k weight gradients of split_beats_library), and
+// the other one-level batches of untransposed products with m, n >= 128, k <=
+// 256, no bias and disjoint outputs (except those that small tiles end before
+// the library begins), go to rocBLAS (atomics off: the same bits on every
+// run); the rest to the small tiles or gemm_kernel (choose_small), and while
+// the library route is switched off (wm_gemm_library) every product
 // to this file's kernels.  A bias is written into C first and the library adds the
 // product to it.  The switch is read once per product; a product racing a
 // switch takes one route or the other, whole.
@@ -1376,25 +1378,32 @@ DmaSplit choose_dma_split(const GemmParams& P, int64_t tiles) {
     return best;
 }
 
-// Whether that beats the library on P, a weight gradient x^T dY over many
-// rows: k is long, and the output's 128 x 128 tiles alone do not fill the chip.
-// The library walks all of k in 64-256 wide tiles there and its rate depends
-// on how those happen to divide the chip: 16-149 TFLOP/s over 60 sizes
-// (m, n from 128 to 4096, k from 512 to 16320), where the split is at
-// 100-131.  Library / split, us: [768, 768] over 4096 62.6 / 59.6,
-// [768, 3072] over 4096 231.6 / 168.2, [1280, 640] over 4416 100.7 / 69.4,
-// [3072, 128] over 8768 420.7 / 75.6, [896, 768] over 10560 143.9 / 124.3,
-// [2048, 1152] over 6208 294.7 / 238.6; the two slower ones of 33 sizes inside
-// the lines are [1152, 896] over 14272 208.7 / 228.4 and [640, 2304] over
-// 9024 207.7 / 222.1.  Outside them the library keeps the product: fewer
-// than 18 tiles ([384, 384] over 6144 30.7 / 35.5), k below 4096 ([768, 1152]
-// over 1408 25.7 / 34.5, [896, 1024] over 3136 48.5 / 61.7), more than 200 tiles
-// ([2560, 1536] over 6400 355.4 / 394.2), and multiples of 64 tiles, which its
-// own tiles divide evenly ([1024, 1024] over 8192 125.4 / 137.9).  A Linear of
-// 4096 x 768 -> 3072, forward and backward, 546.5 -> 497.1 us; attention training
-// at [8, 512, 768] 965 -> 914 us.
+// Whether that beats the library on P, a weight gradient x^T dY over many rows:
+// k is long, and the output's 128 x 128 tiles alone do not fill the chip.  The
+// library's rate there depends on how its own tiles divide the output and on
+// whether it splits k (4-150 TFLOP/s), the split's does not (59-131, more at
+// more tiles and longer k).  Over 8654 sizes drawn at random (m, n 128-6144, k
+// 1024-19136), of the 1839 inside these lines 3 % were more than 3 % slower
+// than the library and the mean is 0.61 of its time:
+//   m >= n: 18 to 191 tiles.  [3072, 768] over 4096 225.7 / 168.1 us, [1280, 640]
+//           over 4416 100.7 / 69.4, [3072, 128] over 8768 420.7 / 75.6, [3584, 384]
+//           over 3392 165.3 / 84.4; the slowest [1152, 768] over 4096 at 1.18;
+//   m < n:  33-48 or 65-80 tiles, or 129-191 with n >= 2.5 m.  [768, 3072] over
+//           4096 231.6 / 168.2.  Between those the library's tiles fit and it is
+//           up to 1.5 times faster ([384, 1280] over 4096, 30 tiles; [256, 2048]
+//           over 5376; [896, 1152] over 4160; [1152, 896] over 14272, where m >= n,
+//           208.7 / 228.4);
+//   multiples of 64 tiles keep the library (12 of 52 slower, [1024, 1024] over
+//           3264 at 1.36), and so do k below 3072 (27 % slower down to 2048), fewer than
+//           18 tiles ([384, 384] over 6144 30.7 / 35.5) and more than 191 ([2560,
+//           1536] over 6400 355.4 / 394.2), though some there would gain ([4096,
+//           896] over 6528 621.7 / 381.9, [2048, 128] over 8512 88.1 / 51.2).
+// A Linear of 4096 x 768 -> 3072, forward and backward, 546.5 -> 497.1 us; attention
+// training at [8, 512, 768] 965 -> 914 us.
 bool split_beats_library(bool ta, bool tb, const GemmParams& P, int64_t tiles) {
-    return ta && !tb && P.k >= 4096 && tiles >= 18 && tiles <= 200 && tiles % 64 != 0;
+    if (!ta || tb || P.k < 3072 || tiles < 18 || tiles > 191 || tiles % 64 == 0) return false;
+    if (P.m >= P.n) return true;
+    return (tiles >= 33 && tiles <= 48) || (tiles >= 65 && tiles <= 80) || (tiles >= 129 && 2 * P.n >= 5 * P.m);
 }
 
 // Whether gemm_dma32_kernel takes P: A transposed, B not, n = 64 (one
@@ -1429,9 +1438,9 @@ int launch_dma32(GemmParams P, int64_t tiles) {
 // S: k steps of one wave; T: tiles of all problems (and k slices), T' in whole
 // rounds of the CUs, T" half way between (a tile's time on a CU shrinks when it
 // is alone there); nk: 32-k stages, 1.5 nk and no 6 for the direct-to-LDS
-// kernels, 0.0135 at unaligned rows, half T" and 3.6 for 64-wide tiles.  c: 1, but from k = 1024 on 1.2, and 2.5 over 48 tiles or
-// more, where neither or both operands are transposed (one is read along k and
-// the other across it).
+// kernels, 0.0135 at unaligned rows, half T" and 3.6 for 64-wide tiles.
+// c: 1, but from k = 1024 on 1.2, and 2.5 over 48 tiles or more, where neither
+// or both operands are transposed (one is read along k, the other across it).
 // A batch that the library takes starts at 7.5 us there; small tiles take it if
 // they end by 6.5.  Over 7285 such products drawn at random, small tiles were
 // chosen where the 128-row kernels or the library are more than 5 % faster 28
