@@ -98,7 +98,7 @@ def test_small_products(wm, m, n, k, batch, ta, tb):
 
 # Weight gradients x^T dY on the k split of the direct-to-LDS kernel (with the library
 # route off; by default the library keeps some): 18 and 200 tiles, equal slices and
-# a shorter last one, and sizes that neither takes whole.
+# a shorter last one, and sizes next to those.
 @pytest.mark.parametrize("m,n,k", [(384, 768, 4096), (768, 384, 4160), (640, 512, 6848), (2560, 1280, 4096),
                                    (384, 768, 4032), (128, 2176, 4096), (1024, 1024, 4096), (384, 768, 4100)])
 @pytest.mark.parametrize("route", [0, 1])
