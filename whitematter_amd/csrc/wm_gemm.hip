@@ -1381,8 +1381,8 @@ DmaSplit choose_dma_split(const GemmParams& P, int64_t tiles) {
 // Whether that beats the library on P, a weight gradient x^T dY over many rows:
 // k is long, and the output's 128 x 128 tiles alone do not fill the chip.  The
 // library's rate there depends on how its own tiles divide the output and on
-// whether it splits k (4-150 TFLOP/s), the split's does not (59-131, more at
-// more tiles and longer k).  Over 8654 sizes drawn at random (m, n 128-6144, k
+// whether it splits k (13-142 TFLOP/s inside the lines, 74 at the median), the
+// split's does not (57-135, 106 at the median, nine in ten over 85).  Over 8654 sizes drawn at random (m, n 128-6144, k
 // 1024-19136), of the 1839 inside these lines 3 % were more than 3 % slower
 // than the library and the mean is 0.61 of its time:
 //   m >= n: 18 to 191 tiles.  [3072, 768] over 4096 225.7 / 168.1 us, [1280, 640]

@@ -14,14 +14,16 @@
 //
 // BatchNorm2d (core/layer.cpp:202-374).  x is [batch, channels, spatial];
 // a channel's elements are `batch` planes of `spatial` contiguous floats.
-// A channel of up to 16384 floats is held in one workgroup's registers: one
-// launch reads it once, reduces it and writes the result.  Larger channels
-// take two passes of (channel, chunk) workgroups that walk the channel's units
-// across plane ends.  Either way the channel's constants are loaded once per
-// workgroup.  The statistics accumulate sum(x) and sum(x^2) (forward) and sum(g),
-// sum(g (x - mean)), sum(x - mean) (backward) in double per thread and per
-// chunk, combined in a fixed order: one pass over the data, no cancellation
-// problem at fp32 data magnitudes, deterministic.
+// A channel of up to 16384 floats (8192 where its units are single floats:
+// planes that are not a multiple of 4, or unaligned) is held in one
+// workgroup's registers: one launch reads it once, reduces it and writes the
+// result.  Larger channels take two passes of (channel, chunk) workgroups that
+// walk the channel's units across plane ends.  Either way the channel's
+// constants are loaded once per workgroup.  The statistics accumulate sum(x)
+// and sum(x^2) (forward) and sum(g), sum(g (x - mean)), sum(x - mean)
+// (backward) in double per thread and per chunk, combined in a fixed order:
+// one pass over the data, no cancellation problem at fp32 data magnitudes,
+// deterministic.
 //
 // MultiHeadAttention's softmax (core/layer.cpp:1198-1237, backward
 // :1343-1360): one row of scores per workgroup with the mask row added in
