@@ -402,6 +402,30 @@ def test_cross_entropy_rows_a_little_longer_than_their_lanes(wm, rows, cols, off
     test_cross_entropy_rows_at_any_alignment(wm, rows, cols, offset)
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(3, 254), (3, 255), (3, 256), (3, 257), (4, 512), (4, 513), (3, 767), (3, 768),
+                                       (3, 769), (2049, 257), (6144, 257), (6145, 257), (6145, 255)])
+def test_cross_entropy_rows_of_single_floats(wm, rows, cols, offset):
+    """Both sides of the widths and row counts between which a written gradient
+    takes a workgroup per row, and rows past its grid."""
+    test_cross_entropy_rows_at_any_alignment(wm, rows, cols, offset)
+
+
+@pytest.mark.parametrize("rows,cols", [(511, 255), (512, 254), (512, 255), (512, 257), (2100, 1023), (513, 4099),
+                                       (9216, 1021), (9300, 1021)])
+def test_nll_backward_rows_of_single_floats(wm, rows, cols):
+    """Both sides of the lines between which a workgroup per row writes the
+    one-hot gradient; nothing written past its end."""
+    lab = ((np.arange(rows) * 7 + cols - 1) % cols).astype(np.float32)
+    dl, dg = wm.DeviceArray.from_host(lab), wm.DeviceArray.from_host(np.float32([0.75]))
+    buf = rng_normal((rows * cols + 8,), seed_of("nll", rows, cols))
+    gx = wm.DeviceArray.from_host(buf)
+    wm.call("wm_nll_bwd", dl.vp, dg.vp, gx.vp, 0, rows, cols)
+    got = gx.to_host()
+    assert oracle.bit_equal(got[:rows * cols].reshape(rows, cols), oracle.get("f32").nll_bwd((rows, cols), lab, 0.75))
+    assert np.array_equal(got[rows * cols:], buf[rows * cols:])
+
+
 def test_cross_entropy_backward_pace(wm):
     """Rows of one float4 more than a workgroup's lanes at some shifts: 1.5 times a
     copy (2.5 with a tile of its own for it)."""

@@ -333,6 +333,28 @@ __global__ void __launch_bounds__(256) head_bwd_ragged_kernel(const float* __res
     }
 }
 
+// A workgroup per row, one float per thread: the few rows whose loads the shifted
+// tiles would leave too few wavefronts to cover.  Bound by latency; [4256, 511]
+// 5.5 us against the tiles' 6.8, [4256, 301] 5.0 against 5.9.
+template <int MODE>
+__global__ void __launch_bounds__(256) head_bwd_row_kernel(const float* __restrict__ x,
+                                                            const float* __restrict__ labels,
+                                                            const float* __restrict__ stats,
+                                                            const float* __restrict__ loss_grad,
+                                                            float* __restrict__ gx, int64_t rows, int64_t cols,
+                                                            float alpha) {
+    const float scale = loss_grad[0] / (float)rows;
+    for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const HeadRow h = head_row<MODE>(stats, labels[r], r, cols, scale);
+        const float* xr = x + r * cols;
+        float* gr = gx + r * cols;
+        for (int64_t c = threadIdx.x; c < cols; c += 256) {
+            const float xv = MODE != kOneHot ? ld_stream1(xr + c) : 0.f;
+            st_stream1(gr + c, head_elem<MODE>(xv, c == h.lab, h, scale, alpha));
+        }
+    }
+}
+
 // NLL: one lane per row.
 __global__ void __launch_bounds__(256) nll_gather_kernel(const float* __restrict__ pred,
                                                           const float* __restrict__ labels, int64_t rows,
@@ -580,12 +602,32 @@ template <int MODE>
 int launch_head_bwd(const float* x, const float* labels, const float* stats, const float* loss_grad, float* gx,
                     int acc, int64_t rows, int64_t cols, float alpha, const char* what) {
     const bool vec = cols % 4 == 0 && aligned16(gx) && (MODE == kOneHot || aligned16(x));
-    const int64_t tiles = (cols / 4 + 255) / 256;
+    const int64_t tiles = (cols / 4 + 255) / 256, cus = num_cus();
+    // A row per workgroup, rows of any alignment.  Up to three passes of single
+    // floats over few enough rows to be bound by latency: up to 24 rows per CU
+    // (4256 rows: 301 classes 5.0 us against 5.9, 511 5.5 against 6.8, but 801 9.0
+    // against 8.5; 6000 rows: 302 5.7 against 6.2, 601 9.5 against 9.6; 8192 rows:
+    // 302 8.3 against 7.5), and up to 12 M elements where the passes are full but
+    // the tiles take one float4 more than their lanes (12000 of 511 13.1 against
+    // 13.9, 24000 of 255 14.7 against 15.8; 32768 of 511 tie, of 767 46.8 against
+    // 43.0).  An accumulated gradient doubles the single loads: 6000 of 479 10.3
+    // against 8.6.
+    // The one-hot gradient only writes and stays in front as long as the L2s about
+    // hold it (32 MB): 4256 rows of 769 4.6 us against 5.7, 12000 of 767 9.7 against
+    // 12.1 and 512 of 10001 5.1 against 5.6, but 1024 of 10001 10.7 against 9.6 and
+    // 32768 of 302 13.0 against 11.5.
+    const bool by_row =
+        cols >= 255 &&
+        (MODE == kOneHot ? rows >= 2 * cus && rows * cols <= (int64_t)9 << 20
+                         : cols < 768 && (rows <= cus * 24 || (cols % 256 == 255 && rows * cols <= (int64_t)12 << 20)));
     // Aligned rows of at least 128 float4s keep a tile of their own: 22.4 us
     // against 29.8 at [16384, 1000].
     if (vec && cols >= 4 * 128 && rows * tiles < ((int64_t)1 << 32)) {
         launch_kernel((head_bwd_tile_kernel<MODE>), dim3(grid_for(rows * tiles, 1, 1 << 12)), dim3(256), 0,
                       stream(), x, labels, stats, loss_grad, gx, acc, rows, cols, alpha);
+    } else if (!vec && !acc && by_row) {
+        launch_kernel((head_bwd_row_kernel<MODE>), dim3((unsigned)std::min<int64_t>(rows, cus * 8)), dim3(256), 0, stream(),
+                      x, labels, stats, loss_grad, gx, rows, cols, alpha);
     } else {
         // Long rows shift to whole 128-byte lines, short ones to 16 bytes.  As
         // many lanes as a row has float4s or a quarter fewer, and one tile up to
@@ -597,7 +639,7 @@ int launch_head_bwd(const float* x, const float* labels, const float* stats, con
         int lg = 0;
         while (lg < 8 && (1 << lg) + (1 << lg) / 4 < (cols + 3) / 4) ++lg;
         const int64_t groups = (rows + (256 >> lg) - 1) / (256 >> lg);
-        const bool more = n4 <= 384;
+        const bool more = n4 > ((int64_t)1 << lg) && n4 <= 384;
         const dim3 grid(more ? 1u : (unsigned)((n4 + 255) / 256), (unsigned)std::min<int64_t>(groups, 65535));
         if (more)
             launch_kernel((head_bwd_ragged_kernel<MODE, true>), grid, dim3(256), 0, stream(), x, labels, stats,
